@@ -333,6 +333,11 @@ __device__ __forceinline__ void load_lds16(const void* src, char* lds_wave_base)
   __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)lds_wave_base, 16, 0, 0);
 }
 
+// The same through a buffer resource: a lane whose offset lies past the resource's end writes zeros to its LDS place.
+__device__ __forceinline__ void buf_lds16(rsrc_t r, uint32_t off, char* lds_wave_base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_wave_base, 16, static_cast<int>(off), 0, 0, 0);
+}
+
 // Wait until at most n vector-memory operations of this wave are outstanding (n a compile-time constant).
 template <int n>
 __device__ __forceinline__ void wait_vmcnt() {

@@ -1366,6 +1366,7 @@ struct MlaPrefillArgs {
   float scale;
   uint16_t* out;  // [nh, dv] per token (token stride out_ts)
   int64_t out_ts;
+  int stored;  // the prompt's rows are in the cache already
 };
 
 __device__ __forceinline__ bool mla_prefill_pos_ok(const MlaPrefillArgs& a, int64_t pos) {
@@ -1388,196 +1389,326 @@ __global__ __launch_bounds__(64) void mla_prefill_store_kernel(MlaPrefillArgs a)
 }
 
 constexpr int kMlaPKeys = 32;  // keys per tile
-constexpr int kMlaPVtRow = 36;  // bf16 per transposed value row in LDS: 32 keys + 4 (72 bytes, see the stores)
 
+// 8 bytes per lane from LDS, transposed within groups of 16 lanes: with lane s of a group reading row s / 4, columns
+// 4 (s % 4) .. + 3 of a 4 x 16 block of bf16, lane i receives column i of the 4 rows (ds_read_b64_tr_b16; the lane layout
+// checked on the device). Four fragments at once, each from place p[i] and `HI` bytes on, waited for in the same block:
+// the builtin makes the compiler wait for every load in flight into LDS, the next tile's among them.
+template <int HI>
+__device__ __forceinline__ void lds_tr4x2(const uint32_t (&p)[4], uint64_t (&lo)[4], uint64_t (&hi)[4]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %2, %9\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %4, %10\n\tds_read_b64_tr_b16 %5, %10 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %6, %11\n\tds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3])
+      : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "n"(HI)
+      : "memory");
+}
 
-// Causal attention of T prompt tokens over the static cache (the new rows already stored): token t at position
-// pos + t takes softmax(scale q_t . K[0..pos+t]^T) . V[0..pos+t] (engine.py:679-682's mask). Grid (T / 16,
-// nh) x NW waves (8 when the grid is small, else 4): a workgroup holds 16 queries of one head, and its waves take
-// the 32-key tiles round robin (wave w: tiles w, w + NW, ...), each keeping its own running max, sum and output for
-// the 16 queries; they are merged through LDS at the end. Per tile, on the 16x16x32 bf16 MFMA:
-//   S^T [32 keys, 16 queries] = K Q^T, the key rows read straight from the cache into A fragments and the
-//     queries held as B fragments (lane: query lane % 16, dims 32 kk + 8 (lane / 16) .. + 7);
+__device__ __forceinline__ uint32_t lds_place(const char* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
+}
+
+__device__ __forceinline__ bf16x8_t lds_frag(const char* p) {
+  return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(p));
+}
+
+// Every LDS read of the wave has returned (and none moves past): its source may be overwritten.
+__device__ __forceinline__ void wait_lgkm0() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (0x7 << 4) | (0 << 8));
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Max over the 4 lanes that share lane % 16.
+__device__ __forceinline__ float quarter_max(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), true, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), true, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// The shape of mla_prefill_attn_kernel: QF 16-query fragments per workgroup, NW waves, head dims up to 32 NKQ (q, k;
+// FULL: exactly) and 16 NT (v).
+template <int QF, int NW, int NKQ, bool FULL, int NT>
+struct MlaP {
+  static constexpr int BQ = 16 * QF;                     // queries per workgroup
+  static constexpr int DVM = 16 * NT;
+  static constexpr int KC = 4 * NKQ, VC = 2 * NT;        // 16-byte chunks of a key, value row in LDS
+  static constexpr int KI = kMlaPKeys * KC / kWave, VI = kMlaPKeys * VC / kWave;  // direct loads per key, value tile
+  static constexpr int K_BYTES = kMlaPKeys * KC * 16, V_BYTES = kMlaPKeys * VC * 16;
+  static constexpr int OROW = DVM + 4;                   // fp32 per output row of the merge
+  static constexpr int ML = BQ * OROW;                   // the wave's max and sum of each query, after its outputs
+  static constexpr int O_BYTES = (ML + 2 * BQ) * 4;
+  static constexpr int WAVE_BYTES = K_BYTES + V_BYTES > O_BYTES ? K_BYTES + V_BYTES : O_BYTES;
+  static constexpr size_t LDS = static_cast<size_t>(NW) * WAVE_BYTES;
+  static_assert(LDS <= 160 * 1024 && KI % 2 == 0, "tile shape");
+};
+
+// The chunk of a tile's row held at LDS place c of the row (an involution). Keys: the 16 rows that a fragment reads at
+// one chunk fall on the 16 distinct 16-byte columns of the banks; values: the 16 rows of a transposing read, 32 bytes
+// each, fall on the 8 columns twice.
+template <int KC>
+__device__ __forceinline__ int mla_k_chunk(int row, int c) {
+  return KC % 16 == 0 ? c ^ (row & 15) : c ^ ((row >> 1) & 7);
+}
+template <int VC>
+__device__ __forceinline__ int mla_v_chunk(int row, int c) {
+  return VC == 16 ? c ^ (2 * (row & 7)) : c ^ (2 * ((row >> 1) & 3));
+}
+
+// Causal attention of T prompt tokens over the static cache: token t at position pos + t takes
+// softmax(scale q_t . K[0..pos+t]^T) . V[0..pos+t] (engine.py:679-682's mask), rows below pos from the cache, the
+// prompt's own from k_new / v_new, which the workgroup of a token's queries also copies to its cache row
+// (engine.py:537-541; no workgroup reads those cache rows, so the copy needs no launch of its own). a.stored: the rows
+// are in the cache already (mla_prefill_store_kernel) and are read there.
+// Grid (nh, query blocks, the last and longest first) x NW waves: with 8 or more heads the workgroups of a head share an
+// XCD, whose L2 then serves its keys and values. A workgroup holds 16 QF queries of one head, and its waves take the
+// 32-key tiles round robin (wave w: tiles w, w + NW, ...; first the cached keys' tiles, then the prompt's), each keeping
+// its own running max, sum and output for all the queries; they are merged through LDS at the end. Per tile, on the
+// 16x16x32 bf16 MFMA:
+//   S^T [32 keys, 16 queries] = K Q^T, the key rows as A fragments, which every query fragment uses, and the queries
+//     held as B fragments (lane: query lane % 16, dims 32 kk + 8 (lane / 16) .. + 7);
 //   the masked softmax update per query is lane-local (a lane of the S^T tiles holds 8 keys of its query
-//     column: 4 (lane / 16) + v and 16 + 4 (lane / 16) + v), the tile max summed over the 4 lane quarters;
+//     column: 4 (lane / 16) + v and 16 + 4 (lane / 16) + v), the tile max taken over the 4 lane quarters;
 //   O^T [dv, 16 queries] += V^T P^T: the B fragment of P comes straight from the S^T registers, its 8 k slots
-//     taking those 8 keys in that order, and the A fragment of V^T (dim lane % 16, the same 8 keys) from a
-//     transposed copy of the value tile the wave stores in its own LDS ([dv][36], two keys per 4-byte store).
+//     taking those 8 keys in that order, and the A fragment of V^T (dim lane % 16, the same 8 keys) by two transposing
+//     reads of the value tile.
+// Bound by the vector-memory path: a tile's 20 KB come by loads straight into the wave's own LDS, the next tile's keys
+// requested as soon as this one's are in registers, its values as soon as this one's are. us per call, 16 heads of
+// 192 / 128, at 500@611, 2000@2000 and 30@3000 (tokens @ position): 59, 588 and 74 with 16 queries per workgroup, tiles
+// by loads into registers and values transposed by stores; 25, 168 and 43 with 32 queries, transposing reads and the
+// next tile in flight, still by register loads (81 at 2000@2000 without the loads); 19.2, 105 and 22 as it is.
 // O^T's lane layout (dims 4 (lane / 16) + v of each 16-dim tile, query lane % 16) keeps the rescaling by the
-// query's exp(m_old - m_new) lane-local as well. Keys past the block's last query are not read (zeros, then
-// masked); queries past T repeat the last token and are not stored. A prompt outside [0, max_len) writes NaN.
-template <int NT, int NW>  // dv <= 16 NT; NW waves per workgroup
-__global__ __launch_bounds__(NW * 64) void mla_prefill_attn_kernel(MlaPrefillArgs a) {
-  constexpr int DVM = 16 * NT;
-  constexpr int VT_BYTES = DVM * kMlaPVtRow * 2;
-  constexpr int MERGE_BYTES = 16 * DVM * 4;  // the wave's O [16 queries][DVM] fp32
-  constexpr int WAVE_BYTES = VT_BYTES > MERGE_BYTES ? VT_BYTES : MERGE_BYTES;
-  __shared__ __align__(16) char s_buf[NW * WAVE_BYTES];
-  __shared__ float s_m[NW][16], s_l[NW][16];
-  const int tid = threadIdx.x, wave = tid / kWave, lane = lane_id();
+// query's exp(m_old - m_new) lane-local as well. Rows past a tile's keys read zero (the buffer resource ends there),
+// and so do the keys past a fragment's last query, so that a value no query of the fragment attends never meets it;
+// queries past T repeat the last token and are not stored. A prompt outside [0, max_len) writes NaN.
+template <int QF, int NW, int NKQ, bool FULL, int NT>
+__global__ __launch_bounds__(NW * 64, 2) void mla_prefill_attn_kernel(MlaPrefillArgs a) {
+  using P = MlaP<QF, NW, NKQ, FULL, NT>;
+  constexpr int BQ = P::BQ, DVM = P::DVM;
+  extern __shared__ __align__(16) char s_mla[];
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lr = lane & 15, lq = lane >> 4;
-  const int h = blockIdx.y, tq0 = blockIdx.x * 16;
+  const int h = blockIdx.x, tq0 = (static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y)) * BQ;
   const int64_t pos = load_pos64(a.pos, a.pos_dtype);
   const int n4 = a.dv / 4;
   if (!mla_prefill_pos_ok(a, pos)) {  // uniform over the workgroup
-    for (int i = tid; i < 16 * a.dv; i += NW * kWave) {
+    for (int i = tid; i < BQ * a.dv; i += NW * kWave) {
       const int t = tq0 + i / a.dv;
       if (t < a.T) a.out[t * a.out_ts + static_cast<int64_t>(h) * a.dv + i % a.dv] = 0x7fc0;  // NaN
     }
     return;
   }
-  const int tlast = min(tq0 + 15, a.T - 1);
-  const int tq = min(tq0 + lr, a.T - 1);
-  const int64_t qlim = pos + tq;          // the keys this lane's query attends: 0 .. qlim
-  const int64_t kend = pos + tlast + 1;   // the keys any query of the workgroup attends: 0 .. kend - 1
-  const int ntiles = static_cast<int>((kend + kMlaPKeys - 1) / kMlaPKeys);
-  const int nkq = (a.dqk + 31) / 32;
-  bf16x8_t qf[8];
-  {
-    const uint16_t* qrow = a.q + tq * a.q_ts + static_cast<int64_t>(h) * a.dqk;
+  const int ctx = static_cast<int>(pos);               // < max_len <= 2^24
+  const int nnew = min(tq0 + BQ, a.T);                 // the prompt's keys that any query of the workgroup attends
+  const int nc = (ctx + kMlaPKeys - 1) / kMlaPKeys, nt_all = nc + (nnew + kMlaPKeys - 1) / kMlaPKeys;
+  // row 0 of each segment and the bytes between rows (the host keeps 32 rows within 2^31 bytes)
+  const uint16_t* kc = a.kc + static_cast<int64_t>(h) * a.max_len * a.dqk;
+  const uint16_t* vc = a.vc + static_cast<int64_t>(h) * a.max_len * a.dv;
+  const uint16_t* kn = a.stored ? kc + pos * a.dqk : a.k_new + static_cast<int64_t>(h) * a.dqk;
+  const uint16_t* vn = a.stored ? vc + pos * a.dv : a.v_new + static_cast<int64_t>(h) * a.dv;
+  const int64_t kn_ts = a.stored ? a.dqk : a.k_ts, vn_ts = a.stored ? a.dv : a.v_ts;
+  char* kt = s_mla + wave * P::WAVE_BYTES;
+  char* vt = kt + P::K_BYTES;
+  // direct load i of a key tile fills LDS chunks 64 i + lane: row krow[i] (+ 16 for the second half), dims kdim[i] ..; of
+  // a value tile row vrow + (64 / VC) i, dims vdim[i % 2] ..
+  constexpr int KH = P::KI / 2, VPI = kWave / P::VC;
+  int krow[KH], kdim[KH], vdim[2];
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
+  for (int i = 0; i < KH; ++i) {
+    krow[i] = (kWave * i + lane) / P::KC;
+    kdim[i] = 8 * mla_k_chunk<P::KC>(krow[i], (kWave * i + lane) % P::KC);
+  }
+  const int vrow = lane / P::VC;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) vdim[i] = 8 * mla_v_chunk<P::VC>(vrow + VPI * i, lane % P::VC);
+  static_assert(P::VC == 16 || P::VC == 8, "value rows: the swizzle repeats after two loads");
+
+  // keys of tile it that exist (0 past the last tile: the loads write zeros and touch no memory)
+  auto rows_of = [&](int it) {
+    return it >= nt_all ? 0 : min(it < nc ? ctx - it * kMlaPKeys : nnew - (it - nc) * kMlaPKeys, kMlaPKeys);
+  };
+  auto load_k = [&](int it) {
+    const bool old = it < nc;
+    const int n = rows_of(it);
+    const int64_t ts = old ? a.dqk : kn_ts, row = n ? static_cast<int64_t>(old ? it : it - nc) * kMlaPKeys : 0;
+    const rsrc_t r = make_rsrc((old ? kc : kn) + row * ts, n ? ((n - 1) * ts + a.dqk) * 2 : 0);
+    const uint32_t ts2 = static_cast<uint32_t>(ts) * 2u;
+#pragma unroll
+    for (int i = 0; i < P::KI; ++i) {
+      const uint32_t off = krow[i % KH] * ts2 + kdim[i % KH] * 2u + (i / KH) * 16u * ts2;
+      buf_lds16(r, (FULL || kdim[i % KH] < a.dqk) ? off : kPast, kt + i * 1024);
+    }
+  };
+  auto load_v = [&](int it) {
+    const bool old = it < nc;
+    const int n = rows_of(it);
+    const int64_t ts = old ? a.dv : vn_ts, row = n ? static_cast<int64_t>(old ? it : it - nc) * kMlaPKeys : 0;
+    const rsrc_t r = make_rsrc((old ? vc : vn) + row * ts, n ? ((n - 1) * ts + a.dv) * 2 : 0);
+    const uint32_t ts2 = static_cast<uint32_t>(ts) * 2u;
+#pragma unroll
+    for (int i = 0; i < P::VI; ++i)
+      buf_lds16(r, vdim[i % 2] < a.dv ? (vrow + VPI * i) * ts2 + vdim[i % 2] * 2u : kPast, vt + i * 1024);
+  };
+  // LDS places of this lane's fragment pieces: key row 16 f + lr, chunk 4 kk + lq; value rows 4 lq + lr / 4 (+ 16),
+  // dims 16 nt + 4 (lr % 4) .. + 3
+  const char* kfrag = kt + lr * P::KC * 16;
+  const int vfr = 4 * lq + lr / 4;
+  const int vplace = vfr * P::VC * 16 + mla_v_chunk<P::VC>(vfr, (lr % 4) / 2) * 16 + (lr & 1) * 8;
+
+  bf16x8_t qf[QF][NKQ];
+#pragma unroll
+  for (int f = 0; f < QF; ++f) {
+    const uint16_t* qrow = a.q + min(tq0 + 16 * f + lr, a.T - 1) * a.q_ts + static_cast<int64_t>(h) * a.dqk;
+#pragma unroll
+    for (int kk = 0; kk < NKQ; ++kk) {
       const int d = 32 * kk + 8 * lq;
-      uint4 x = make_uint4(0, 0, 0, 0);
-      if (kk < nkq && d < a.dqk) x = *reinterpret_cast<const uint4*>(qrow + d);
-      qf[kk] = __builtin_bit_cast(bf16x8_t, x);
+      const bool ok = FULL || d < a.dqk;
+      qf[f][kk] = __builtin_bit_cast(bf16x8_t, and_mask16(*reinterpret_cast<const uint4*>(qrow + (ok ? d : 0)), ok));
     }
   }
-  floatx4 o[NT];
+  floatx4 o[QF][NT];
+  float m[QF], l[QF];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) o[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
-  uint16_t* vt = reinterpret_cast<uint16_t*>(s_buf + wave * WAVE_BYTES);
-  const int64_t hk = static_cast<int64_t>(h) * a.max_len;
-  constexpr int RV = (DVM + 31) / 32;  // value pieces (2 keys x 8 dims) per lane: 16 key pairs x dv / 8 groups
-  const int ndg = a.dv / 8;
-  for (int kt = wave; kt < ntiles; kt += NW) {
-    const int64_t j0 = static_cast<int64_t>(kt) * kMlaPKeys;
-    // every load of the tile first, unconditionally (rows and dims past the ends read the row's first piece and are
-    // zeroed after), so the tile costs one trip to memory: where each load sat behind its own range test, the
-    // compiler waited for each before the next (16 round trips per tile)
-    // value tile: lane piece i = lane + 64 r -> key pair kp = i % 16, dim group dg = i / 16
-    uint4 va[RV], vb[RV];
-    bool oka[RV], okb[RV];
+  for (int f = 0; f < QF; ++f) {
+    m[f] = -INFINITY;
+    l[f] = 0.f;
 #pragma unroll
-    for (int r = 0; r < RV; ++r) {
-      const int i = lane + kWave * r, kp = i % 16, dg = i / 16;
-      const int64_t ja = j0 + 2 * kp;
-      const bool dok = dg < ndg;
-      oka[r] = dok && ja < kend;
-      okb[r] = dok && ja + 1 < kend;
-      va[r] = *reinterpret_cast<const uint4*>(a.vc + (hk + (oka[r] ? ja : 0)) * a.dv + (oka[r] ? 8 * dg : 0));
-      vb[r] = *reinterpret_cast<const uint4*>(a.vc + (hk + (okb[r] ? ja + 1 : 0)) * a.dv + (okb[r] ? 8 * dg : 0));
-    }
-    uint4 kx[2][8];
+    for (int nt = 0; nt < NT; ++nt) o[f][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float sc = a.scale * 1.4426950408889634f;  // scores in units of log2: exp2 gives the weights
+  wait_vmcnt<0>();  // the queries: from here on only the tiles' loads are in flight
+  load_k(wave);
+  load_v(wave);
+  for (int it = wave; it < nt_all; it += NW) {
+    const int n = rows_of(it);
+    const bool old = it < nc;
+    const int j0 = (it - nc) * kMlaPKeys;  // the tile's first prompt token (prompt tiles)
+    wait_vmcnt<P::VI>();  // the tile's keys (its values still in flight)
+    wave_lds_fence();
+    bf16x8_t kx[2][NKQ];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const int64_t j = j0 + 16 * n + lr;
-      const bool live = j < kend;
-      const uint16_t* krow = a.kc + (hk + (live ? j : 0)) * a.dqk;
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const int d = 32 * kk + 8 * lq;
-        const bool ok = live && d < a.dqk;
-        kx[n][kk] = and_mask16(*reinterpret_cast<const uint4*>(krow + (ok ? d : 0)), ok);
+      for (int kk = 0; kk < NKQ; ++kk)
+        kx[u][kk] = lds_frag(kfrag + u * 16 * P::KC * 16 + mla_k_chunk<P::KC>(lr, 4 * kk + lq) * 16);
+    wait_lgkm0();  // read before the next tile overwrites them
+    load_k(it + NW);
+    floatx4 s[QF][2];
+#pragma unroll
+    for (int f = 0; f < QF; ++f) s[f][0] = s[f][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < NKQ; ++kk)  // 2 QF independent sums in turn
+#pragma unroll
+      for (int f = 0; f < QF; ++f)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          s[f][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kx[u][kk], qf[f][kk], s[f][u], 0, 0, 0);
+    // masked online softmax: slot e < 4 is key 4 lq + e of the tile, slot e >= 4 key 16 + 4 lq + e - 4
+    bf16x8_t pf[QF];
+#pragma unroll
+    for (int f = 0; f < QF; ++f) {
+      const int lim = old ? n : min(n, tq0 + 16 * f + lr - j0 + 1);  // keys of the tile this lane's query attends
+      float sv[8];
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int key = e < 4 ? 4 * lq + e : 16 + 4 * lq + e - 4;
+        const float x = e < 4 ? s[f][0][e] : s[f][1][e - 4];
+        sv[e] = key < lim ? x * sc : -INFINITY;
+        tmax = fmaxf(tmax, sv[e]);
+      }
+      const float mn = fmaxf(m[f], quarter_max(tmax));
+      const float mu = mn == -INFINITY ? 0.f : mn;  // a query with no key yet in this wave's tiles
+      const float alpha = exp2_fast(m[f] - mu);
+      m[f] = mn;
+      float ps = 0.f;
+      uint32_t pw[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p0 = exp2_fast(sv[2 * e] - mu), p1 = exp2_fast(sv[2 * e + 1] - mu);
+        ps += p0 + p1;
+        pw[e] = static_cast<uint32_t>(f32_to_bf16(p0)) | (static_cast<uint32_t>(f32_to_bf16(p1)) << 16);
+      }
+      l[f] = fmaf(l[f], alpha, ps);
+      pf[f] = __builtin_bit_cast(bf16x8_t, make_uint4(pw[0], pw[1], pw[2], pw[3]));
+      if (__any(alpha != 1.f)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) o[f][nt] *= alpha;
       }
     }
+    const bool diag = QF > 1 && !old && j0 == tq0;  // keys 16 .. 31 lie past every query of the first fragment
+    wait_vmcnt<P::KI>();  // the tile's values (the next tile's keys still in flight)
+    wave_lds_fence();
 #pragma unroll
-    for (int r = 0; r < RV; ++r) {
-      va[r] = and_mask16(va[r], oka[r]);
-      vb[r] = and_mask16(vb[r], okb[r]);
-    }
-    floatx4 s[2];
+    for (int n0 = 0; n0 < NT; n0 += 4) {
+      uint32_t place[4];
+      uint64_t lo[4], hi[4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      s[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < 4; ++b) place[b] = lds_place(vt) + (vplace ^ (32 * (n0 + b)));
+      lds_tr4x2<16 * P::VC * 16>(place, lo, hi);
+      if (n0 + 4 == NT) load_v(it + NW);  // the tile's last values are read
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk)
-        if (kk < nkq)
-          s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kx[n][kk]), qf[kk], s[n], 0, 0, 0);
-    }
-    // the transposed value tile: dword (dim 8 dg + e, keys 2 kp, 2 kp + 1); 16 consecutive key pairs per dim
-    // row and 4 dim groups 8 x 18 dwords apart per store keep the 64 lanes on distinct banks
-    wave_lds_fence();  // the previous tile's reads of vt are done
+      for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int r = 0; r < RV; ++r) {
-      const int i = lane + kWave * r, kp = i % 16, dg = i / 16;
-      if (dg < ndg) {
-        const uint32_t xa[4] = {va[r].x, va[r].y, va[r].z, va[r].w}, xb[4] = {vb[r].x, vb[r].y, vb[r].z, vb[r].w};
-        auto* dst = reinterpret_cast<uint32_t*>(vt) + (8 * dg) * (kMlaPVtRow / 2) + kp;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          dst[(2 * e) * (kMlaPVtRow / 2)] = __builtin_amdgcn_perm(xb[e], xa[e], 0x05040100u);      // low halves
-          dst[(2 * e + 1) * (kMlaPVtRow / 2)] = __builtin_amdgcn_perm(xb[e], xa[e], 0x07060302u);  // high halves
+        for (int f = 0; f < QF; ++f) {
+          const uint64_t hf = (f == 0 && diag) ? 0 : hi[b];
+          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, make_uint4(static_cast<uint32_t>(lo[b]), static_cast<uint32_t>(lo[b] >> 32),
+                                                                      static_cast<uint32_t>(hf), static_cast<uint32_t>(hf >> 32)));
+          o[f][n0 + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[f], o[f][n0 + b], 0, 0, 0);
         }
-      }
-    }
-    // masked online softmax: slot e < 4 is key j0 + 4 lq + e, slot e >= 4 key j0 + 16 + 4 lq + e - 4
-    float sv[8];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int64_t key = j0 + (e < 4 ? 4 * lq + e : 16 + 4 * lq + e - 4);
-      const float x = e < 4 ? s[0][e] : s[1][e - 4];
-      sv[e] = key <= qlim ? x * a.scale : -INFINITY;
-      tmax = fmaxf(tmax, sv[e]);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-    const float mn = fmaxf(m, tmax);
-    const float mu = mn == -INFINITY ? 0.f : mn;  // a query with no key yet in this wave's tiles
-    const float alpha = __expf(m - mu);
-    m = mn;
-    float ps = 0.f;
-    uint32_t pw[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float p0 = __expf(sv[2 * e] - mu), p1 = __expf(sv[2 * e + 1] - mu);
-      ps += p0 + p1;
-      pw[e] = static_cast<uint32_t>(f32_to_bf16(p0)) | (static_cast<uint32_t>(f32_to_bf16(p1)) << 16);
-    }
-    l = fmaf(l, alpha, ps);
-    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pw[0], pw[1], pw[2], pw[3]));
-    wave_lds_fence();  // the stores of vt before the loads
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      o[nt] *= alpha;
-      if (16 * nt < a.dv) {
-        const uint16_t* row = vt + (16 * nt + lr) * kMlaPVtRow;
-        const uint2 lo = *reinterpret_cast<const uint2*>(row + 4 * lq);
-        const uint2 hi = *reinterpret_cast<const uint2*>(row + 16 + 4 * lq);
-        o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y)),
-                                                        pf, o[nt], 0, 0, 0);
-      }
     }
   }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  // the wave's state into its own LDS region (its value tile is no longer read), then the merge
+  // this workgroup's tokens into their cache rows
+  if (!a.stored) {
+    const int kp = a.dqk / 8, np = kp + a.dv / 8, rows = nnew - tq0;
+    for (int i = tid; i < rows * np; i += NW * kWave) {
+      const int t = i / np, c = i % np;
+      const bool isk = c < kp;
+      const int64_t row = pos + tq0 + t;
+      const uint16_t* src = isk ? kn + (tq0 + t) * kn_ts + 8 * c : vn + (tq0 + t) * vn_ts + 8 * (c - kp);
+      uint16_t* dst = isk ? a.kc + (static_cast<int64_t>(h) * a.max_len + row) * a.dqk + 8 * c
+                          : a.vc + (static_cast<int64_t>(h) * a.max_len + row) * a.dv + 8 * (c - kp);
+      *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
+    }
+  }
+  // the wave's state into its own LDS region (the loads past its last tile done), then the merge
+  wait_vmcnt<0>();
   wave_lds_fence();
-  float* so = reinterpret_cast<float*>(s_buf + wave * WAVE_BYTES);
+  float* so = reinterpret_cast<float*>(s_mla + wave * P::WAVE_BYTES);
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-    if (16 * nt < a.dv) *reinterpret_cast<floatx4*>(so + lr * DVM + 16 * nt + 4 * lq) = o[nt];
-  if (lq == 0) {
-    s_m[wave][lr] = m;
-    s_l[wave][lr] = l;
+  for (int f = 0; f < QF; ++f) {
+    l[f] += __shfl_xor(l[f], 16, kWave);
+    l[f] += __shfl_xor(l[f], 32, kWave);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      *reinterpret_cast<floatx4*>(so + (16 * f + lr) * P::OROW + 16 * nt + 4 * lq) = o[f][nt];
+    if (lq == 0) {
+      so[P::ML + 16 * f + lr] = m[f];
+      so[P::ML + BQ + 16 * f + lr] = l[f];
+    }
   }
   __syncthreads();
-  for (int i = tid; i < 16 * n4; i += NW * kWave) {
+  for (int i = tid; i < BQ * n4; i += NW * kWave) {
     const int qi = i / n4, d = 4 * (i % n4), t = tq0 + qi;
     if (t >= a.T) continue;
-    float mx = s_m[0][qi];  // finite: wave 0 holds key 0
+    auto state = [&](int w) { return reinterpret_cast<const float*>(s_mla + w * P::WAVE_BYTES); };
+    float mx = state(0)[P::ML + qi];  // finite: wave 0 holds key 0
 #pragma unroll
-    for (int w = 1; w < NW; ++w) mx = fmaxf(mx, s_m[w][qi]);
+    for (int w = 1; w < NW; ++w) mx = fmaxf(mx, state(w)[P::ML + qi]);
     float lt = 0.f;
     floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float wt = __expf(s_m[w][qi] - mx);
-      lt = fmaf(s_l[w][qi], wt, lt);
-      acc += wt * *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(s_buf + w * WAVE_BYTES) +
-                                                    qi * DVM + d);
+      const float wt = exp2_fast(state(w)[P::ML + qi] - mx);
+      lt = fmaf(state(w)[P::ML + BQ + qi], wt, lt);
+      acc += wt * *reinterpret_cast<const floatx4*>(state(w) + qi * P::OROW + d);
     }
     const float inv = 1.f / lt;
     uint16_t* dst = a.out + t * a.out_ts + static_cast<int64_t>(h) * a.dv + d;
@@ -1585,6 +1716,31 @@ __global__ __launch_bounds__(NW * 64) void mla_prefill_attn_kernel(MlaPrefillArg
     const uint32_t w1 = static_cast<uint32_t>(f32_to_bf16(acc[2] * inv)) | (static_cast<uint32_t>(f32_to_bf16(acc[3] * inv)) << 16);
     *reinterpret_cast<uint2*>(dst) = make_uint2(w0, w1);
   }
+}
+
+template <int QF, int NW, int NKQ, bool FULL, int NT>
+int launch_mla_prefill(const MlaPrefillArgs& a, hipStream_t st) {
+  using P = MlaP<QF, NW, NKQ, FULL, NT>;
+  auto kern = mla_prefill_attn_kernel<QF, NW, NKQ, FULL, NT>;
+  int rc = mm::allow_lds(kern, P::LDS, "mla_prefill_attn");
+  if (rc) return rc;
+  const dim3 grid(static_cast<unsigned>(a.nh), static_cast<unsigned>((a.T + P::BQ - 1) / P::BQ));
+  hipLaunchKernelGGL(kern, grid, dim3(NW * kWave), P::LDS, st, a);
+  return mm::check_launch("mla_prefill_attn");
+}
+
+// The workgroup's shape by how many there would be of 32 queries, against the CUs. us per call at 16 heads of 192 / 128
+// (tokens @ position), 32 queries on half a CU's waves | 16 queries on half | 16 queries on all:
+//   2000@2000 114 | 158 | 179, 1024@0 21.8 | 25.0 | 32.3   more than a CU each: 32 queries share every key tile read
+//   500@611 20.8 | 20.5 | 23.2, 300@0 11.3 | 8.8 | 11.3    every CU still gets a workgroup of 16 queries
+//   256@1000 20.2 | 14.1 | 13.1, 30@3000 37.5 | 26.5 | 22.2  few workgroups: more waves share a query block's tiles
+template <int NKQ, bool FULL, int NT>
+int launch_mla_prefill_shape(const MlaPrefillArgs& a, hipStream_t st) {
+  constexpr int NW = NKQ <= 6 ? 8 : 6;  // waves whose tiles fill one CU's LDS
+  const int64_t cus = mm::cu_count(), wgs = static_cast<int64_t>((a.T + 31) / 32) * a.nh;
+  if (wgs > cus) return launch_mla_prefill<2, NW / 2, NKQ, FULL, NT>(a, st);
+  if (2 * wgs > cus) return launch_mla_prefill<1, NW / 2, NKQ, FULL, NT>(a, st);
+  return launch_mla_prefill<1, NW, NKQ, FULL, NT>(a, st);
 }
 
 template <int K>
@@ -1950,19 +2106,16 @@ extern "C" int mm_mla_prefill_attn(const void* q, int64_t q_ts, const void* k_ne
   a.out = static_cast<uint16_t*>(out);
   a.out_ts = out_ts;
   hipStream_t st = MM_STREAM(stream);
-  hipLaunchKernelGGL(mla_prefill_store_kernel, dim3(static_cast<unsigned>(T), static_cast<unsigned>(nh)), dim3(kWave),
-                     0, st, a);
-  int rc = mm::check_launch("mla_prefill_attn store");
-  if (rc) return rc;
-  const dim3 grid(static_cast<unsigned>((T + 15) / 16), static_cast<unsigned>(nh));
-  // fewer workgroups than two per CU: 8 waves each, so that each wave walks half as many key tiles
-  const bool wide = static_cast<int64_t>(grid.x) * grid.y < 2 * mm::cu_count();
-  if (dv <= 64) {
-    if (wide) hipLaunchKernelGGL((mla_prefill_attn_kernel<4, 8>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((mla_prefill_attn_kernel<4, 4>), grid, dim3(256), 0, st, a);
-  } else {
-    if (wide) hipLaunchKernelGGL((mla_prefill_attn_kernel<8, 8>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((mla_prefill_attn_kernel<8, 4>), grid, dim3(256), 0, st, a);
+  // the attention kernel addresses a tile's 32 rows by 32-bit offsets; token strides past that (2^25 elements) store the
+  // rows first and read them from the cache
+  a.stored = k_ts >= (1 << 25) || v_ts >= (1 << 25);
+  if (a.stored) {
+    hipLaunchKernelGGL(mla_prefill_store_kernel, dim3(static_cast<unsigned>(T), static_cast<unsigned>(nh)), dim3(kWave),
+                       0, st, a);
+    int rc = mm::check_launch("mla_prefill_attn store");
+    if (rc) return rc;
   }
-  return mm::check_launch("mla_prefill_attn");
+  if (dv <= 64)
+    return dqk == 192 ? launch_mla_prefill_shape<6, true, 4>(a, st) : launch_mla_prefill_shape<8, false, 4>(a, st);
+  return dqk == 192 ? launch_mla_prefill_shape<6, true, 8>(a, st) : launch_mla_prefill_shape<8, false, 8>(a, st);
 }

@@ -379,6 +379,53 @@ def test_mla_prefill_rows_past_the_prompt_are_never_read_and_out_of_range_writes
         assert torch.isnan(out.float()).all() and torch.equal(kc, k0) and torch.equal(vc, v0)
 
 
+@pytest.mark.parametrize("nh,dq,dv,T,pos", [
+    (16, 192, 128, 33, 31), (16, 192, 128, 15, 32), (16, 192, 128, 32, 33), (16, 192, 128, 257, 1), (16, 192, 128, 545, 64),
+    (9, 192, 64, 31, 95), (16, 192, 64, 300, 5), (16, 192, 64, 530, 0), (3, 248, 120, 49, 63), (16, 256, 128, 290, 17),
+    (16, 136, 8, 530, 40), (2, 192, 16, 17, 0)])
+def test_mla_prefill_tiles_and_shapes(nh, dq, dv, T, pos):
+    """Query blocks of 16 and 32, waves per workgroup, key tiles of the cache and of the prompt that end inside, at and
+    past a tile, and head dims below the padded ones: outputs and caches against the oracle."""
+    print(f"[mla prefill tiles] nh={nh} dq={dq} dv={dv} T={T} pos={pos}", flush=True)
+    L = pos + T + 3
+    kc = W.normal((1, nh, L, dq), 1.0, 530, DEV)
+    vc = W.normal((1, nh, L, dv), 1.0, 531, DEV)
+    kc[:, :, pos:], vc[:, :, pos:] = float("nan"), float("inf")  # rows the prompt fills, and rows past it
+    k0, v0 = kc.clone(), vc.clone()
+    q, kn, vn = _prompt(nh, dq, dv, T, 532)
+    out = TA.mla_prefill_attn(q, kn, vn, kc, vc, torch.tensor([pos], device=DEV))
+    ro, rk, rv = A.mla_prefill_attn(q.reshape(T, nh, dq).cpu(), kn.reshape(T, nh, dq).cpu(),
+                                    vn.reshape(T, nh, dv).cpu(), k0[0].cpu(), v0[0].cpu(), pos)
+    close(out.reshape(T, nh, dv), ro)
+    assert torch.equal(kc[0, :, :pos + T].cpu(), rk[:, :pos + T]) and torch.equal(vc[0, :, :pos + T].cpu(), rv[:, :pos + T])
+    assert torch.isnan(kc[:, :, pos + T:]).all() and torch.isinf(vc[:, :, pos + T:]).all()
+
+
+def test_mla_prefill_values_past_a_query_block_and_far_token_strides():
+    """An infinite value row reaches no query of the 16-query blocks before it (32 queries share a workgroup here); tokens
+    2^25 elements apart take the path that stores the rows first and equal the same prompt packed, bit for bit."""
+    nh, dq, dv, T, pos = 16, 192, 128, 544, 10
+    kc = W.normal((1, nh, T + pos, dq), 1.0, 540, DEV)
+    vc = W.normal((1, nh, T + pos, dv), 1.0, 541, DEV)
+    q, kn, vn = _prompt(nh, dq, dv, T, 542)
+    vn.view(T, nh, dv)[80] = float("inf")
+    print("[mla prefill inf]", flush=True)
+    out = TA.mla_prefill_attn(q, kn, vn, kc, vc, torch.tensor([pos], device=DEV)).float()
+    assert torch.isfinite(out[:80]).all() and not torch.isfinite(out[80:96]).any()
+    nh, T, L = 2, 3, 40
+    q, kn, vn = _prompt(nh, dq, dv, T, 543)
+    far_k, far_v = (torch.zeros((T - 1) * 2 ** 25 + nh * d, device=DEV, dtype=BF).as_strided((T, nh * d), (2 ** 25, 1))
+                    for d in (dq, dv))
+    far_k.copy_(kn.reshape(T, -1))
+    far_v.copy_(vn.reshape(T, -1))
+    ke, ve = W.normal((1, nh, L, dq), 1.0, 544, DEV), W.normal((1, nh, L, dv), 1.0, 545, DEV)
+    kf, vf = ke.clone(), ve.clone()
+    p = torch.tensor([33], device=DEV)
+    print("[mla prefill far strides]", flush=True)
+    assert torch.equal(TA.mla_prefill_attn(q, kn, vn, ke, ve, p), TA.mla_prefill_attn(q, far_k, far_v, kf, vf, p))
+    assert torch.equal(ke, kf) and torch.equal(ve, vf)
+
+
 def test_mla_prefill_one_token_equals_decode_and_graph_replays_follow_the_position():
     nh, dq, dv, L = 16, 192, 128, 512
     kc = W.normal((1, nh, L, dq), 1.0, 520, DEV)
