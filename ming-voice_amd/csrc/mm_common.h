@@ -296,6 +296,11 @@ __device__ __forceinline__ uint4 buf16(rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
 }
 
+// With a wave-uniform part of the offset, which costs no vector instruction.
+__device__ __forceinline__ float4 buf16f(rsrc_t r, uint32_t off, uint32_t uniform) {
+  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), static_cast<int>(uniform), 0));
+}
+
 __device__ __forceinline__ uint32_t buf4(rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(off), 0, 0));
 }

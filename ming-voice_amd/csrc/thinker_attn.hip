@@ -42,6 +42,18 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The LDS address of a pointer into shared memory, as LDS instructions take it.
+__device__ __forceinline__ uint32_t lds_place(const char* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
+}
+
+// Every LDS read of the wave has returned (and none moves past): its source may be overwritten.
+__device__ __forceinline__ void wait_lgkm0() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (0x7 << 4) | (0 << 8));
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------------------------------------------------- KDA
 
 struct KdaArgs {
@@ -409,272 +421,497 @@ __global__ __launch_bounds__(64 * NWB) void kda_recurrent_kernel(KdaArgs a, cons
 // (per-channel products taken directly, never as ratios, so a strong decay underflows to zero instead of 0 / 0):
 //   k_t . (the decayed state before token t's write) = a_t + sum_{j<t} A[t][j] u_j,
 //       a_t = (k_t P_t) . S0,  A[t][j] = sum_c k_tc k_jc D(j, t)_c
-//   u_t = beta_t (v_t - a_t - sum_{j<t} A[t][j] u_j)        (forward substitution, j in order)
+//   u_t = beta_t (v_t - a_t - sum_{j<t} A[t][j] u_j), that is u = M (v - a) with the lower triangular
+//       M = (I + diag(beta) A)^-1 diag(beta), found row by row by forward substitution
 //   o_t = q_t . S_t = b_t + sum_{j<=t} B[t][j] u_j,
 //       b_t = (q_t P_t) . S0,  B[t][j] = sum_c q_tc k_jc D(j, t)_c (j < t),  B[t][t] = q_t . k_t
 //   S_end = P_{C-1} S0 + sum_j (k_j D(j, C-1)) u_j^T
 // Everything but S0 and v depends on the head alone, not on the value columns: kda_chunk_prep_kernel computes it
 // for every (chunk, head) at once into a block of the workspace; kda_chunk_kernel then carries its value columns'
-// state from chunk to chunk, and no token waits for a sum over k of the token before it. Padding tokens (past
-// n_valid, or past T in the last chunk) have decay 1 and beta 0, so their u is 0 and the state passes them unchanged.
+// state from chunk to chunk. All products run on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: lane l gives
+// row l % 16 and k l / 16 of A, column l % 16 and k l / 16 of B, and gets rows 4 (l / 16) + v of column l % 16), with
+// the k order of each step chosen so that every result is the next product's operand as it stands: k step s takes
+// k = 4 (l / 16) + s. Padding tokens (past n_valid, or past T in the last chunk) have decay 1, beta 0 and v - a taken
+// as 0, so their u is 0 and the state passes them unchanged.
+//
+// us per call at 16 heads of 128 x 128, 32 / 64 / 192 / 512 / 700 / 2048 tokens: 12.2 / 14.3 / 21.9 / 43.7 / 57.8 / 146
+// (0.85 a chunk, of which the 28 matrix instructions on the longest path are 0.4, and 10 .. 40 the preparation); 16.9 /
+// 21.8 / 39.5 / 85.7 / 116 / 315 with the pair sums and the sums over k on the vector units and the substitution across
+// lanes. The state's error against 64 bits over those lengths is 9 .. 14 % smaller than either other form's, its 16
+// terms a chunk being summed on their own.
 
-// A (chunk, head) block of the workspace, in floats: k P [C][K], q P [C][K], W = k D(., C-1) [C][K], P_{C-1} [K],
-// A [C][C] with beta_t on its diagonal, B [C][C] (zero above the diagonal).
+// A (chunk, head) block of the workspace, in floats, each operand in the order of its lanes (one 16-byte piece a lane):
+// k P, q P [K / 16][lane][4] (token lane % 16, channels 16 tile + 4 (lane / 16) ..), W = (k D(., C-1))^T [K / 16][lane][4]
+// (channel 16 tile + lane % 16, tokens 4 (lane / 16) ..), P_{C-1} [K], M [C][C], B [C][C] (zero above the diagonal).
 template <int K>
 struct KdaBlk {
   static constexpr int C = kKdaChunk;
-  static constexpr int KP = 0, QP = C * K, W = 2 * C * K, PC = 3 * C * K, A = PC + K, B = A + C * C;
+  static constexpr int KP = 0, QP = C * K, W = 2 * C * K, PC = 3 * C * K, M = PC + K, B = M + C * C;
   static constexpr int SIZE = B + C * C;
   static_assert(SIZE % 4 == 0, "blocks stay 16-byte aligned");
 };
 
-// 32 values over the 64 lanes of a wave: x[0] becomes the wave's total of value lane % 32 (the halves summed by
-// v_permlane32_swap, then transposed over the rows and within them: 63 exchanges, against 192 for 32 separate sums).
-__device__ __forceinline__ void wave_sums32(float (&x)[32]);
+__device__ __forceinline__ floatx4 mfma4(float x, float y, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+}
 
-// Grid (chunks, H) x 16 waves. Wave w prepares token w of the chunk (kda_prep_token: q and k normalised, the decay,
-// beta, q . k; a token past T gets q = k = 0, decay 1, beta 0) into LDS, then writes its rows: k P, q P and W of token
-// w (the decay products over the other tokens' channels read back from LDS, taken as predicated products so that no
-// register array is indexed at run time), P_{C-1} (wave C-1), and row w of A and B (entry j a wave sum over the
-// channels, the 32 entries summed together by wave_sums32).
-template <int K>
-__global__ __launch_bounds__(64 * kKdaChunk) void kda_chunk_prep_kernel(KdaArgs a, float* __restrict__ blk) {
+// The sum over the 4 lanes that share lane % 16.
+__device__ __forceinline__ float quarter_sum(float v) { return half_pair_sum(row_pair_sum(v)); }
+
+// 8 consecutive bf16 or fp32 values; VEC: their address is 16-byte aligned.
+template <bool VEC, bool F32>
+__device__ __forceinline__ void ld8(const void* base, int64_t i, float (&x)[8]) {
+  if constexpr (F32) {
+    const float* p = static_cast<const float*>(base) + i;
+    if constexpr (VEC) {
+      const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 4);
+      x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w, x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = p[e];
+    }
+  } else {
+    const uint16_t* p = static_cast<const uint16_t*>(base) + i;
+    if constexpr (VEC) {
+      const uint4 r = *reinterpret_cast<const uint4*>(p);
+      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[2 * e] = bf_lo(w[e]), x[2 * e + 1] = bf_hi(w[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = bf16_to_f32(p[e]);
+    }
+  }
+}
+
+// x[0..3] of the 4 lanes of a quad, transposed: lane i of the quad gets value i of lanes 0 .. 3.
+__device__ __forceinline__ float4 quad_transpose(const float* x) {
+  const int lane = lane_id();
+  const bool b0 = lane & 1, b1 = lane & 2;
+  const float s0 = dpp_f32<kDppXor1>(b0 ? x[0] : x[1]), s1 = dpp_f32<kDppXor1>(b0 ? x[2] : x[3]);
+  const float y0 = b0 ? s0 : x[0], y1 = b0 ? x[1] : s0, y2 = b0 ? s1 : x[2], y3 = b0 ? x[3] : s1;
+  const float t0 = dpp_f32<kDppXor2>(b1 ? y0 : y2), t1 = dpp_f32<kDppXor2>(b1 ? y1 : y3);
+  return make_float4(b1 ? t0 : y0, b1 ? t1 : y1, b1 ? y2 : t0, b1 ? y3 : t1);
+}
+
+// Grid (chunks H, heads within a chunk) x K / 32 waves. Wave p holds channels 32 p .. + 31 of the chunk: lane l token l % 16, channels
+// 32 p + 8 (l / 16) .. + 7. The decay products between pairs of tokens split by the highest bit in which the pair
+// differs: for t in the upper and j in the lower half of a block of 2^(L+1) tokens, D(j, t) is the product over the rest
+// of j's half times that over t's half up to t, so with F_L = that part for each token, level L's pairs are
+// (k F_L) (k F_L)^T and (q F_L) (k F_L)^T on the matrix units; the halves' products double from level to level by lane
+// exchanges, and after the last they are P and D(., C-1). The waves' parts meet in LDS, wave L (and L + 2 when there are
+// two) summing level L. VEC: q, k, g, dt_bias by 16-byte loads; GF32: g is fp32.
+template <int K, bool VEC, bool GF32>
+__global__ __launch_bounds__(2 * K, 3) void kda_chunk_prep_kernel(KdaArgs a, float* __restrict__ blk) {
   using L = KdaBlk<K>;
-  constexpr int C = L::C, NJ = K / kWave;
-  __shared__ float s_k[C][K], s_d[C][K];
-  const int ci = blockIdx.x, h = blockIdx.y;
-  const int w = threadIdx.x / kWave, lane = lane_id();
-  const int t0 = ci * C;
-  const bool in = t0 + w < a.T;
-  float qn[NJ], kn[NJ], dv[NJ], beta, qk;
-  kda_prep_token<K>(a, in ? t0 + w : t0, h, t0 + w >= kda_valid(a), qn, kn, dv, beta, qk);
+  constexpr int C = L::C, NW = K / 32, AR = C + 4;
+  __shared__ __align__(16) float s_A[C * AR];
+  __shared__ __align__(16) float s_beta[C];
+  __shared__ float s_qk[NW][C], s_nq[NW][C], s_nk[NW][C];
+  __shared__ floatx4 s_acc[4][2][NW][kWave];
+  const int p = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
+  const int ci = blockIdx.x / a.H, h = blockIdx.x % a.H;
+  const int t = lane & 15, g = lane >> 4;
+  const int64_t row = min(ci * C + t, a.T - 1), ch = static_cast<int64_t>(h) * K + 32 * p + 8 * g;
+  const bool in = ci * C + t < a.T, pad = ci * C + t >= kda_valid(a);
+  float q[8], k[8], d[8], dt[8];
+  ld8<VEC, false>(a.q, row * a.q_ts + ch, q);
+  ld8<VEC, false>(a.k, row * a.k_ts + ch, k);
+  ld8<VEC, GF32>(a.g, row * a.g_ts + ch, d);
+  if (a.use_gate) ld8<VEC, true>(a.dt_bias, ch, dt);
+  float beta = ld_any(a.beta, a.beta_dtype, row * a.b_ts + h);
+  const float nA = a.use_gate ? __expf(a.A_log[h]) : 0.f;
+  float sq = 0.f, sk = 0.f;
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    qn[j] = in ? qn[j] : 0.f;
-    kn[j] = in ? kn[j] : 0.f;
-    dv[j] = in ? dv[j] : 1.f;
-    s_k[w][lane + kWave * j] = kn[j];
-    s_d[w][lane + kWave * j] = dv[j];
+  for (int e = 0; e < 8; ++e) {
+    sq = fmaf(q[e], q[e], sq);
+    sk = fmaf(k[e], k[e], sk);
   }
-  beta = in ? beta : 0.f;
-  qk = in ? qk : 0.f;
+  sq = quarter_sum(sq);
+  sk = quarter_sum(sk);
+  if (g == 0) s_nq[p][t] = sq, s_nk[p][t] = sk;
+  // one branch on the gate's form for all 8, none within
+  if (a.use_gate && isnan(a.lower_bound)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = d[e] + dt[e], y = log1pf(__expf(fminf(x, 20.f)));
+      d[e] = -nA * (x > 20.f ? x : y);
+    }
+  } else if (a.use_gate) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d[e] = a.lower_bound / (1.f + __expf(-nA * (d[e] + dt[e])));
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) d[e] = in && !pad ? __expf(d[e]) : 1.f;
   __syncthreads();
-  // P_w = d_0 ... d_w and R_w = D(w, C-1) = d_{w+1} ... d_{C-1}; then, j running down, D(j, w) = d_{j+1} ... d_w
-  float P[NJ], R[NJ], D[NJ];
+  float qs = a.scale, ks = 1.f;
+  if (a.use_l2norm) {
+    sq = s_nq[0][t] + s_nq[1][t];
+    sk = s_nk[0][t] + s_nk[1][t];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) P[j] = R[j] = D[j] = 1.f;
-  float x[32];  // the lane's parts of A[w][j] (x[j]) and B[w][j] (x[16 + j]), j < w
-#pragma unroll
-  for (int s2 = C - 1; s2 >= 0; --s2) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const float ds = s_d[s2][lane + kWave * j];
-      P[j] = s2 <= w ? P[j] * ds : P[j];
-      R[j] = s2 > w ? R[j] * ds : R[j];
-    }
+    for (int w = 2; w < NW; ++w) sq += s_nq[w][t], sk += s_nk[w][t];
+    qs = a.scale / sqrtf(sq + 1e-6f);
+    ks = 1.f / sqrtf(sk + 1e-6f);
   }
+  float qk = 0.f;
+  float pre[8], suf[8], tot[8];
 #pragma unroll
-  for (int jj = C - 1; jj >= 0; --jj) {
-    float sa = 0.f, sb = 0.f;
+  for (int e = 0; e < 8; ++e) {
+    q[e] = in ? q[e] * qs : 0.f;
+    k[e] = in ? k[e] * ks : 0.f;
+    qk = fmaf(q[e], k[e], qk);
+    pre[e] = tot[e] = d[e];
+    suf[e] = 1.f;
+  }
+  qk = quarter_sum(qk);
+  if (g == 0) s_qk[p][t] = qk;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int ch = lane + kWave * j;
-      if (jj + 1 < C) D[j] = jj + 1 <= w ? D[j] * s_d[jj + 1][ch] : D[j];
-      const float kd = s_k[jj][ch] * D[j];
-      sa = fmaf(kn[j], kd, sa);
-      sb = fmaf(qn[j], kd, sb);
+  for (int lv = 0; lv < 4; ++lv) {
+    const bool up = (t >> lv) & 1;
+    floatx4 accA = floatx4{0.f, 0.f, 0.f, 0.f}, accB = accA;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float f = up ? pre[e] : suf[e];
+      const float x = k[e] * f, y = q[e] * f;
+      accA = mfma4(x, x, accA);
+      accB = mfma4(y, x, accB);
+      // the other half's product (the same in all its lanes)
+      const float o = lv == 0 ? dpp_f32<kDppXor1>(tot[e]) : lv == 1 ? dpp_f32<kDppXor2>(tot[e])
+                    : lv == 2 ? dpp_f32<kDppHalfMirror>(tot[e]) : dpp_f32<kDppMirror>(tot[e]);
+      pre[e] = up ? pre[e] * o : pre[e];
+      suf[e] = up ? suf[e] : suf[e] * o;
+      tot[e] *= o;
     }
-    x[jj] = jj < w ? sa : 0.f;
-    x[C + jj] = jj < w ? sb : 0.f;
+    s_acc[lv][0][p][lane] = accA;
+    s_acc[lv][1][p][lane] = accB;
   }
   float* out = blk + (static_cast<int64_t>(ci) * a.H + h) * L::SIZE;
+  const int tile = 2 * p + g / 2;
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int ch = lane + kWave * j;
-    out[L::KP + w * K + ch] = kn[j] * P[j];
-    out[L::QP + w * K + ch] = qn[j] * P[j];
-    out[L::W + w * K + ch] = kn[j] * R[j];
-    if (w == C - 1) out[L::PC + ch] = P[j];
+  for (int e = 0; e < 8; e += 4) {  // channels 8 (g % 2) + e .. of the tile
+    const int at = (tile * kWave + 16 * (2 * (g % 2) + e / 4) + t) * 4;
+    *reinterpret_cast<float4*>(out + L::KP + at) =
+        make_float4(k[e] * pre[e], k[e + 1] * pre[e + 1], k[e + 2] * pre[e + 2], k[e + 3] * pre[e + 3]);
+    *reinterpret_cast<float4*>(out + L::QP + at) =
+        make_float4(q[e] * pre[e], q[e + 1] * pre[e + 1], q[e + 2] * pre[e + 2], q[e + 3] * pre[e + 3]);
+    const float w[4] = {k[e] * suf[e], k[e + 1] * suf[e + 1], k[e + 2] * suf[e + 2], k[e + 3] * suf[e + 3]};
+    *reinterpret_cast<float4*>(out + L::W + (tile * kWave + 16 * (t / 4) + 8 * (g % 2) + e + t % 4) * 4) = quad_transpose(w);
+    if (t == 0)
+      *reinterpret_cast<float4*>(out + L::PC + 32 * p + 8 * g + e) = make_float4(tot[e], tot[e + 1], tot[e + 2], tot[e + 3]);
   }
-  wave_sums32(x);
-  if (lane < 2 * C) {
-    const int jj = lane % C;
-    const float diag = lane < C ? beta : qk;
-    out[(lane < C ? L::A : L::B) + w * C + jj] = jj < w ? x[0] : jj == w ? diag : 0.f;
+  if (p == 0 && g == 0) {
+    if (a.beta_logits) beta = 1.f / (1.f + __expf(-beta));
+    s_beta[t] = in && !pad ? beta : 0.f;
   }
-}
-
-// Transposed sums over the lanes of a column. In a step the two lanes of a pair each keep the half of their values
-// whose index has their lane bit, adding the partner's copy of it; the pairs are those of group_sum (v_permlane16_swap
-// across rows of 16 for lane bit 4, then the DPP mirror, half mirror, xor 2 and xor 1 for bits 3 .. 0: a partner
-// differs in the step's bit and agrees in every bit split before), so the lane's last value sums all the lanes.
-// One step of 16-lane sums on x[0 .. 2H): pairs (v, v + H) split on lane bit `bit`.
-template <int ctrl, int H>
-__device__ __forceinline__ void col_step(float* x, int bit) {
-  const bool hi = (lane_id() >> bit) & 1;
+  __syncthreads();
+  // rows 4 g + v, column t of A and B: the level of the pair's highest differing bit
+  for (int lv = p; lv < 4; lv += NW) {
+    floatx4 x = s_acc[lv][0][0][lane] + s_acc[lv][0][1][lane], y = s_acc[lv][1][0][lane] + s_acc[lv][1][1][lane];
 #pragma unroll
-  for (int v = 0; v < H; ++v) {
-    const float keep = hi ? x[v + H] : x[v], send = hi ? x[v] : x[v + H];
-    x[v] = keep + dpp_f32<ctrl>(send);
-  }
-}
-
-// 16 values over the 16 lanes of a row: x[0] becomes the row's total of value lane % 16 (15 exchanges, against 64
-// for 16 separate sums).
-__device__ __forceinline__ void row_sums16(float* x) {
-  col_step<kDppMirror, 8>(x, 3);
-  col_step<kDppHalfMirror, 4>(x, 2);
-  col_step<kDppXor2, 2>(x, 1);
-  col_step<kDppXor1, 1>(x, 0);
-}
-
-__device__ __forceinline__ void wave_sums32(float (&x)[32]) {
+    for (int w = 2; w < NW; ++w) x += s_acc[lv][0][w][lane], y += s_acc[lv][1][w][lane];
 #pragma unroll
-  for (int v = 0; v < 32; ++v) x[v] = half_pair_sum(x[v]);
+    for (int v = 0; v < 4; ++v) {
+      const int r = 4 * g + v;
+      if ((r ^ t) >> lv == 1) {
+        s_A[r * AR + t] = x[v];
+        out[L::B + r * C + t] = r > t ? y[v] : 0.f;
+      } else if (lv == 0 && r == t) {
+        float z = s_qk[0][t] + s_qk[1][t];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 16]), false, false);
-    x[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  row_sums16(x);
-}
-
-// 32 values over the RG lanes of a column: RG = 32, x[0] = total of value rg; RG = 16, x[0] and x[16] = totals of
-// values rg and 16 + rg.
-template <int RG>
-__device__ __forceinline__ void column_sums(float (&x)[32]) {
-  if constexpr (RG == 32) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {  // row 0 keeps v, row 1 keeps v + 16, both at index v
-      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 16]), false, false);
-      x[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        for (int w = 2; w < NW; ++w) z += s_qk[w][t];
+        out[L::B + r * C + t] = z;
+      }
     }
-    row_sums16(x);
-  } else {
-    row_sums16(x);
-    row_sums16(x + 16);
+  }
+  __syncthreads();
+  if (p > 0) return;
+  // column t of M, row after row (every lane group the same), every row of A read before the first is used
+  float m[C];
+  float4 ar[C][C / 4];
+#pragma unroll
+  for (int r = 1; r < C; ++r)
+#pragma unroll
+    for (int j = 0; 4 * j < r; ++j) ar[r][j] = *reinterpret_cast<const float4*>(s_A + r * AR + 4 * j);
+  float bt[C];
+#pragma unroll
+  for (int r = 0; r < C; r += 4) {
+    const float4 b = *reinterpret_cast<const float4*>(s_beta + r);
+    bt[r] = b.x, bt[r + 1] = b.y, bt[r + 2] = b.z, bt[r + 3] = b.w;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < C; ++r) {
+    float x = r == t ? 1.f : 0.f;
+#pragma unroll
+    for (int j = 0; j < r; ++j) {
+      const float4& q4 = ar[r][j / 4];
+      x = fmaf(j % 4 == 0 ? -q4.x : j % 4 == 1 ? -q4.y : j % 4 == 2 ? -q4.z : -q4.w, m[j], x);
+    }
+    m[r] = bt[r] * x;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float lo = g & 1 ? m[4 + v] : m[v], hi = g & 1 ? m[12 + v] : m[8 + v];
+    out[L::M + (4 * g + v) * C + t] = g & 2 ? hi : lo;
   }
 }
 
-// Grid (V / COLS, H) x NWB waves, the layout of kda_recurrent_kernel: lane (c = lane / RG, rg = lane % RG) holds
-// state rows 4 rg .. 4 rg + 3 of one value column. A chunk's block comes into LDS by global_load_lds (two buffers,
-// the next chunk loading during this one). Per chunk a lane forms its parts of a_t and b_t for the 16 tokens and the
-// column's lanes sum them transposed, so that one lane holds a_t ("A lane" of token t) and one b_t ("B lane"; for
-// RG = 32 lanes 0-15 and 16-31, for RG = 16 every lane is both). The forward substitution then runs across the
-// lanes: at step j the A lane of token j has all of its terms, forms u_j = beta_j r_j, and u_j goes to the column's
-// lanes by readlane; every A lane of a later token subtracts A[t][j] u_j, every B lane adds B[t][j] u_j. Each lane
-// keeps the 16 u for its rows of the state update; the B lanes store the outputs.
-template <int K, int NWB>
-__global__ __launch_bounds__(64 * NWB) void kda_chunk_kernel(KdaArgs a, const float* __restrict__ blk) {
+// A barrier for LDS accesses only: the wave's own are done, its global and direct loads stay in flight (a fence would
+// wait for the direct ones).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// 16-byte reads of LDS filled by direct loads (already waited for), waited for in the same block: for an ordinary read
+// the compiler waits until no direct load is in flight.
+__device__ __forceinline__ floatx4 lds_read(uint32_t p) {
+  floatx4 x;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(x) : "v"(p) : "memory");
+  return x;
+}
+// The operands of a worker's chunk at p (lane's place; KdaLds offsets) but k P, which is the next chunk's, at pn.
+template <int TPW>
+__device__ __forceinline__ void lds_read_chunk(uint32_t p, uint32_t ppc, uint32_t pm, uint32_t pn, floatx4 (&qp)[TPW],
+                                               floatx4 (&wt)[TPW], floatx4 (&pc)[TPW], floatx4& m, floatx4 (&kp)[TPW]) {
+  if constexpr (TPW == 2)
+    asm volatile(
+        "ds_read_b128 %0, %9 offset:2048\n\tds_read_b128 %1, %9 offset:3072\n\t"
+        "ds_read_b128 %6, %11\n\t"
+        "ds_read_b128 %4, %10\n\tds_read_b128 %5, %10 offset:64\n\t"
+        "ds_read_b128 %2, %9 offset:4096\n\tds_read_b128 %3, %9 offset:5120\n\t"
+        "ds_read_b128 %7, %12\n\tds_read_b128 %8, %12 offset:1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(qp[0]), "=&v"(qp[1]), "=&v"(wt[0]), "=&v"(wt[1]), "=&v"(pc[0]), "=&v"(pc[1]), "=&v"(m), "=&v"(kp[0]), "=&v"(kp[1])
+        : "v"(p), "v"(ppc), "v"(pm), "v"(pn)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %5 offset:1024\n\tds_read_b128 %3, %7\n\tds_read_b128 %2, %6\n\t"
+        "ds_read_b128 %1, %5 offset:2048\n\tds_read_b128 %4, %8\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(qp[0]), "=&v"(wt[0]), "=&v"(pc[0]), "=&v"(m), "=&v"(kp[0])
+        : "v"(p), "v"(ppc), "v"(pm), "v"(pn)
+        : "memory");
+}
+
+// Operands in LDS of kda_chunk_kernel: each worker wave's of kDepth chunks (its tiles of k P, q P, W, then P_{C-1} and
+// M), then the output wave's B.
+template <int K>
+struct KdaLds {
+  static constexpr int TPW = K / 64, kDepth = 4;                      // state tiles (16 rows) per wave; chunks in flight
+  static constexpr int KP = 0, QP = TPW * 1024, W = 2 * TPW * 1024, PC = 3 * TPW * 1024, M = PC + 1024, STAGE = M + 1024;
+  static constexpr int B = 4 * kDepth * STAGE;
+  static constexpr size_t BYTES = B + kDepth * 1024;
+  static constexpr int LOADS = 3 * TPW + 2;                           // direct loads per chunk of a worker, besides v
+};
+
+// Grid (H, V / 16) x 5 waves (with 8 or more heads, a head's workgroups share an XCD and its L2): 16 value columns of one
+// head. Waves 0 .. 3 hold K / 4 state rows each (the matrix instruction's result layout), form their parts of a and b,
+// exchange the parts of a through LDS (one barrier a chunk) and update their rows; wave 4 forms the outputs of the chunk
+// before from the parts of b and wave 0's u. The operands come by direct loads into each wave's own LDS, three chunks
+// ahead: a chunk's 26 KB would take longer than its products through register loads. FAR: rows of v (or o) too far apart
+// for 32-bit offsets.
+template <int K, bool FAR>
+__global__ __launch_bounds__(320) void kda_chunk_kernel(KdaArgs a, const float* __restrict__ blk) {
   using L = KdaBlk<K>;
-  constexpr int C = L::C, RPL = 4, RG = K / RPL, CPW = kWave / RG, COLS = NWB * CPW;
-  constexpr int NT = NWB * kWave, UNITS = L::SIZE / 4, NU = (UNITS + NT - 1) / NT;
-  constexpr int VPT = (C * COLS + NT - 1) / NT;
-  constexpr bool DUAL = RG == C;  // every lane both an A and a B lane
-  static_assert((RG == 32 || RG == 16) && C == 16, "column lanes");
-  // separate arrays, so that a chunk's LDS reads need not wait for the next chunk's loads into the other one
-  __shared__ __align__(16) float s_b0[L::SIZE], s_b1[L::SIZE];
-  __shared__ float s_v0[C][COLS], s_v1[C][COLS];
-  const int h = blockIdx.y, tid = threadIdx.x, wave = tid / kWave, lane = lane_id();
-  const int c = lane / RG, rg = lane % RG, r0 = RPL * rg;
-  const int64_t V = a.V;
-  const int64_t col0 = static_cast<int64_t>(blockIdx.x) * COLS;
-  const int cw = wave * CPW + c;
-  const int tA = rg % C;                       // token of the lane's A role (RG = 32: lanes rg < 16)
-  const bool isA = DUAL || rg < C, isB = DUAL || rg >= C;
-  float* st = a.state + static_cast<int64_t>(h) * K * V + col0 + cw;
-  float S[RPL];
-#pragma unroll
-  for (int i = 0; i < RPL; ++i) S[i] = st[static_cast<int64_t>(r0 + i) * V];
+  using S_ = KdaLds<K>;
+  constexpr int C = L::C, TPW = S_::TPW, kDepth = S_::kDepth;
+  constexpr int LOADS = S_::LOADS + 4;  // and the chunk's 4 values of v
+  extern __shared__ __align__(16) char s_kda[];
+  // the parts of a and b and u, of two chunks: arrays of their own, or the compiler makes each store to them wait for
+  // the direct loads in flight
+  __shared__ float4 s_a[2][4][kWave], s_b[2][4][kWave], s_u[2][kWave];
+  const int h = blockIdx.x, lane = lane_id(), t16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t V = a.V, col = static_cast<int64_t>(blockIdx.y) * 16 + t16;
+  const int64_t colc = min(col, V - 1);  // columns past V (V a multiple of 8) repeat the last one and are not stored
   const int nch = (a.T + C - 1) / C;
-  const float* bh = blk + static_cast<int64_t>(h) * L::SIZE;
   const int64_t cs = static_cast<int64_t>(a.H) * L::SIZE;  // between the chunks of a head
-  uint16_t rv[VPT];  // raw bf16 v, converted once the chunk's loads are waited for
-  auto issue = [&](int ci, float* dst) {
-#pragma unroll
-    for (int j = 0; j < NU; ++j) {
-      const int u = tid + NT * j;
-      if (u < UNITS) load_lds16(bh + ci * cs + u * 4, reinterpret_cast<char*>(dst) + (wave * kWave + NT * j) * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) {  // rows past the prompt (never used: beta 0) load its last token's row
-      const int i = tid + NT * j, tt = min(ci * C + i / COLS, a.T - 1);
-      rv[j] = a.v[tt * a.v_ts + static_cast<int64_t>(h) * V + col0 + i % COLS];
-    }
+  const float* bh = blk + static_cast<int64_t>(h) * L::SIZE;
+  const uint32_t lane16 = lane * 16u, row16 = t16 * (C * 4u) + g * 16u;
+  auto at4 = [](const float4& x, int s) { return s == 0 ? x.x : s == 1 ? x.y : s == 2 ? x.z : x.w; };
+  auto f4 = [](const floatx4& x) { return make_float4(x[0], x[1], x[2], x[3]); };
+  auto sum4 = [&](const float4 (*p)[kWave]) {  // of the four waves' parts
+    const float4 x = p[0][lane], y = p[1][lane], z = p[2][lane], u = p[3][lane];
+    return floatx4{((x.x + y.x) + z.x) + u.x, ((x.y + y.y) + z.y) + u.y, ((x.z + y.z) + z.z) + u.z, ((x.w + y.w) + z.w) + u.w};
   };
-  // u_j of this lane's column: the value of its lane j (j wave-uniform)
-  auto col_bcast = [&](float x, int j) {
-    float r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__float_as_int(x), j));
+  // chunks past the last give the last one's block
+  auto block = [&](int ci) { return make_rsrc(bh + min(ci, nch - 1) * cs, L::SIZE * 4); };
+  // Runs chunk(ci, j) over all chunks (j = ci % kDepth), whole groups of kDepth, then the rest, the first kDepth - 1
+  // chunks' loads issued before; chunk(ci, ..) issues those of chunk ci + kDepth - 1.
+  auto run = [&](auto issue, auto first, auto chunk) {
 #pragma unroll
-    for (int cc = 1; cc < CPW; ++cc) {
-      const float o = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__float_as_int(x), cc * RG + j));
-      r = c == cc ? o : r;
-    }
-    return r;
+    for (int j = 0; j < kDepth - 1; ++j) issue(j, j);
+    first();
+    int c0 = 0;
+    for (; c0 + kDepth <= nch; c0 += kDepth)
+#pragma unroll
+      for (int j = 0; j < kDepth; ++j) chunk(c0 + j, j);
+#pragma unroll
+    for (int j = 0; j < kDepth - 1; ++j)
+      if (c0 + j < nch) chunk(c0 + j, j);
+    lds_barrier();
   };
-  auto chunk = [&](int ci, const float* in, float (*vb)[COLS], float* in_next) {
-    wait_vmcnt<0>();
+  if (wave < 4) {
+    const int nvalid = kda_valid(a);
+    const uint16_t* vh = a.v + static_cast<int64_t>(h) * V;
+    uint32_t voff[4];
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const int i = tid + NT * j;
-      if (i < C * COLS) vb[i / COLS][i % COLS] = bf16_to_f32(rv[j]);
-    }
-    if constexpr (NWB == 1) wave_lds_fence(); else __syncthreads();
-    if (ci + 1 < nch) issue(ci + 1, in_next);
-    float x[32];  // the lane's parts of a_t (x[t]) and b_t (x[16 + t])
+    for (int v = 0; v < 4; ++v) voff[v] = static_cast<uint32_t>((4 * g + v) * a.v_ts + colc) * 2u;
+    char* own = s_kda + wave * kDepth * S_::STAGE;
+    floatx4 S[TPW];
+    float* st = a.state + (static_cast<int64_t>(h) * K + 16 * wave * TPW + 4 * g) * V + colc;
 #pragma unroll
-    for (int t = 0; t < C; ++t) {
-      const float4 kp = *reinterpret_cast<const float4*>(in + L::KP + t * K + r0);
-      const float4 qp = *reinterpret_cast<const float4*>(in + L::QP + t * K + r0);
-      x[t] = fmaf(kp.x, S[0], kp.y * S[1]) + fmaf(kp.z, S[2], kp.w * S[3]);
-      x[C + t] = fmaf(qp.x, S[0], qp.y * S[1]) + fmaf(qp.z, S[2], qp.w * S[3]);
-    }
-    column_sums<RG>(x);  // RG = 32: x[0] = a_rg or b_(rg-16); RG = 16: x[0] = a_rg, x[16] = b_rg
-    // the lane's rows of A and B (A's diagonal holds beta)
-    const float* arow = in + L::A + tA * C;
-    const float* brow = in + L::B + (DUAL ? rg : (rg >= C ? rg - C : 0)) * C;
-    float ca[C], cb[C];
+    for (int i = 0; i < TPW; ++i)
 #pragma unroll
-    for (int j = 0; j < C; j += 4) {
-      const float4 av = *reinterpret_cast<const float4*>(arow + j);
-      const float4 bv = *reinterpret_cast<const float4*>(brow + j);
-      ca[j] = av.x, ca[j + 1] = av.y, ca[j + 2] = av.z, ca[j + 3] = av.w;
-      cb[j] = bv.x, cb[j + 1] = bv.y, cb[j + 2] = bv.z, cb[j + 3] = bv.w;
-    }
-    const float beta = arow[tA];
-    float ra = isA ? vb[tA][cw] - x[0] : 0.f;  // v_t - a_t, less the earlier u's terms as they come
-    float rb = DUAL ? x[16] : x[0];            // b_t, plus B[t][j] u_j
-    float uall[C];
+      for (int v = 0; v < 4; ++v) S[i][v] = st[(16 * i + v) * V];
+    uint16_t rv[kDepth][4];
+    // a chunk's loads in three parts of 4 or so, issued between the matrix instructions of another chunk: 12 at once
+    // hold the wave up for longer than they are worth
+    constexpr int PART1 = 2 * TPW;
+    auto issue1 = [&](int ci, int j) {
+      const rsrc_t b = block(ci);
+      char* d = own + j * S_::STAGE;
 #pragma unroll
-    for (int j = 0; j < C; ++j) {
-      uall[j] = col_bcast(ra * beta, j);
-      ra = tA > j ? fmaf(-ca[j], uall[j], ra) : ra;
-      rb = fmaf(cb[j], uall[j], rb);
-    }
-    const float4 pc = *reinterpret_cast<const float4*>(in + L::PC + r0);
-    S[0] *= pc.x;
-    S[1] *= pc.y;
-    S[2] *= pc.z;
-    S[3] *= pc.w;
+      for (int i = 0; i < TPW; ++i) {
+        const uint32_t tile = (wave * TPW + i) * 1024u + lane16;
+        buf_lds16(b, L::KP * 4 + tile, d + S_::KP + i * 1024);
+        buf_lds16(b, L::QP * 4 + tile, d + S_::QP + i * 1024);
+      }
+    };
+    auto issue2 = [&](int ci, int j) {
+      const rsrc_t b = block(ci);
+      char* d = own + j * S_::STAGE;
 #pragma unroll
-    for (int j = 0; j < C; ++j) {
-      const float4 wv = *reinterpret_cast<const float4*>(in + L::W + j * K + r0);
-      S[0] = fmaf(wv.x, uall[j], S[0]);
-      S[1] = fmaf(wv.y, uall[j], S[1]);
-      S[2] = fmaf(wv.z, uall[j], S[2]);
-      S[3] = fmaf(wv.w, uall[j], S[3]);
+      for (int i = 0; i < TPW; ++i)
+        buf_lds16(b, L::W * 4 + (wave * TPW + i) * 1024u + lane16, d + S_::W + i * 1024);
+      buf_lds16(b, L::PC * 4 + lane16, d + S_::PC);  // its K channels, then the start of M
+      buf_lds16(b, L::M * 4 + lane16, d + S_::M);
+    };
+    auto issue3 = [&](int ci, int j) {
+      if constexpr (FAR) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rv[j][v] = vh[min(ci * C + 4 * g + v, a.T - 1) * a.v_ts + colc];
+      } else {
+        const int n = min(a.T - ci * C, C);
+        const rsrc_t r = make_rsrc(vh + static_cast<int64_t>(ci) * C * a.v_ts, n > 0 ? ((n - 1) * a.v_ts + V) * 2 : 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rv[j][v] = __builtin_amdgcn_raw_buffer_load_b16(r, static_cast<int>(voff[v]), 0, 0);
+      }
+    };
+    auto issue = [&](int ci, int j) {
+      issue1(ci, j);
+      issue2(ci, j);
+      issue3(ci, j);
+    };
+    // The matrix pipe takes 32 cycles an instruction (28 of them a chunk), so the order is fixed: while the parts of a
+    // are exchanged it works on b.
+    const uint32_t mine = lds_place(own) + lane16, mpc = lds_place(own) + S_::PC + wave * TPW * 64 + g * 16,
+                   mm = lds_place(own) + S_::M + row16;
+    floatx4 kp[TPW];
+    auto first = [&] {  // k P of chunk 0
+      wait_vmcnt<(kDepth - 2) * LOADS>();
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) kp[i] = lds_read(mine + S_::KP + i * 1024);
+    };
+    auto chunk = [&](int ci, int j) {
+      floatx4 as[TPW], bs[TPW], sc[TPW], qp[TPW], wt[TPW], pc[TPW], kn[TPW], m;
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) as[i] = bs[i] = sc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) as[i] = mfma4(kp[i][s], S[i][s], as[i]);
+      __builtin_amdgcn_sched_barrier(0);
+      const int ni = ci + kDepth - 1, nj = (j + kDepth - 1) % kDepth;  // its place was the last chunk's, all read
+      issue1(ni, nj);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt<(kDepth - 3) * LOADS + PART1>();  // this chunk and the next are in LDS
+      const uint32_t at_j = j * S_::STAGE;
+      lds_read_chunk<TPW>(mine + at_j, mpc + at_j, mm + at_j, mine + (j + 1) % kDepth * S_::STAGE, qp, wt, pc, m, kn);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (TPW == 2) as[0] += as[1];
+      s_a[ci & 1][wave][lane] = f4(as[0]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) bs[i] = mfma4(qp[i][0], S[i][0], bs[i]);
+      lds_barrier();
+      const floatx4 at = sum4(s_a[ci & 1]);
+#pragma unroll
+      for (int s = 1; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) bs[i] = mfma4(qp[i][s], S[i][s], bs[i]);
+      __builtin_amdgcn_sched_barrier(0);
+      issue2(ni, nj);
+      __builtin_amdgcn_sched_barrier(0);
+      // u = M (v - a), by every wave
+      floatx4 u = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        u = mfma4(m[s], 4 * g + s < nvalid - ci * C ? bf16_to_f32(rv[j][s]) - at[s] : 0.f, u);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) sc[i] = mfma4(wt[i][s], u[s], sc[i]);
+      __builtin_amdgcn_sched_barrier(0);
+      issue3(ni, nj);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        // the chunk's 16 terms are summed on their own, so that the state is rounded once a chunk
+#pragma unroll
+        for (int v = 0; v < 4; ++v) S[i][v] = fmaf(S[i][v], pc[i][v], sc[i][v]);
+        kp[i] = kn[i];
+      }
+      if constexpr (TPW == 2) bs[0] += bs[1];
+      s_b[ci & 1][wave][lane] = f4(bs[0]);
+      if (wave == 0) s_u[ci & 1][lane] = f4(u);
+    };
+    run(issue, first, chunk);
+    if (col < V) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) st[(16 * i + v) * V] = S[i][v];
     }
-    const int t = ci * C + (DUAL ? rg : rg - C);
-    if (isB && t < a.T) a.o[t * a.o_ts + static_cast<int64_t>(h) * V + col0 + cw] = f32_to_bf16(rb);
-    if constexpr (NWB == 1) wave_lds_fence();  // the chunk's reads before the loads two chunks on
-  };
-  issue(0, s_b0);
-  for (int ci = 0; ci < nch; ci += 2) {
-    chunk(ci, s_b0, s_v0, s_b1);
-    if (ci + 1 < nch) chunk(ci + 1, s_b1, s_v1, s_b0);
+  } else {
+    auto issue = [&](int ci, int j) { buf_lds16(block(ci), L::B * 4 + lane16, s_kda + S_::B + j * 1024); };
+    uint16_t* oh = a.o + static_cast<int64_t>(h) * V;
+    uint32_t ooff[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) ooff[v] = col < V ? static_cast<uint32_t>((4 * g + v) * a.o_ts + col) * 2u : kPast;
+    floatx4 b1 = floatx4{0.f, 0.f, 0.f, 0.f};  // B of the chunk before
+    const uint32_t mine = lds_place(s_kda + S_::B) + row16;
+    auto outputs = [&](int ci) {
+      floatx4 o = sum4(s_b[ci & 1]);
+      const float4 u = s_u[ci & 1][lane];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) o = mfma4(b1[s], at4(u, s), o);
+      if constexpr (FAR) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int t = ci * C + 4 * g + v;
+          if (t < a.T && col < V) oh[t * a.o_ts + col] = f32_to_bf16(o[v]);
+        }
+      } else {  // rows past T lie past the resource
+        const int n = min(a.T - ci * C, C);
+        const rsrc_t r = make_rsrc(oh + static_cast<int64_t>(ci) * C * a.o_ts, ((n - 1) * a.o_ts + V) * 2);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(o[v]), r, static_cast<int>(ooff[v]), 0, 0);
+      }
+    };
+    auto chunk = [&](int ci, int j) {
+      issue(ci + kDepth - 1, (j + kDepth - 1) % kDepth);
+      lds_barrier();
+      // the chunk's B: three later blocks and, from the fourth chunk on, three chunks' stores may be in flight
+      if (ci < kDepth) wait_vmcnt<kDepth - 1>();
+      else wait_vmcnt<5 * (kDepth - 1)>();
+      const floatx4 b = lds_read(mine + j * 1024);
+      if (ci > 0) outputs(ci - 1);
+      b1 = b;
+    };
+    run(issue, [] {}, chunk);
+    outputs(nch - 1);
   }
-#pragma unroll
-  for (int i = 0; i < RPL; ++i) st[static_cast<int64_t>(r0 + i) * V] = S[i];
 }
 
 // ----------------------------------------------------------------------------------------- short conv
@@ -1407,19 +1644,8 @@ __device__ __forceinline__ void lds_tr4x2(const uint32_t (&p)[4], uint64_t (&lo)
       : "memory");
 }
 
-__device__ __forceinline__ uint32_t lds_place(const char* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
-}
-
 __device__ __forceinline__ bf16x8_t lds_frag(const char* p) {
   return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(p));
-}
-
-// Every LDS read of the wave has returned (and none moves past): its source may be overwritten.
-__device__ __forceinline__ void wait_lgkm0() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (0x7 << 4) | (0 << 8));
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -1765,24 +1991,31 @@ int launch_kda(const KdaArgs& a, float* ws, hipStream_t st) {
   return mm::check_launch("kda_recurrent");
 }
 
-// The chunked form: token preparation, the (chunk, head) blocks after the token rows, then the chunk recurrence.
+// The chunked form: the (chunk, head) blocks, then the chunks in turn.
+template <int K, bool VEC, bool GF32>
+int launch_kda_prep(const KdaArgs& a, float* blk, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>((a.T + kKdaChunk - 1) / kKdaChunk) * a.H));
+  hipLaunchKernelGGL((kda_chunk_prep_kernel<K, VEC, GF32>), grid, dim3(2 * K), 0, st, a, blk);
+  return mm::check_launch("kda_chunk prep");
+}
+
 template <int K>
 int launch_kda_chunk(const KdaArgs& a, float* ws, hipStream_t st) {
   if (a.T <= kKdaShortT) return launch_kda<K>(a, ws, st);  // a decode step: one launch, no workspace
-  float* blk = ws;
-  const unsigned nch = static_cast<unsigned>((a.T + kKdaChunk - 1) / kKdaChunk);
-  hipLaunchKernelGGL((kda_chunk_prep_kernel<K>), dim3(nch, static_cast<unsigned>(a.H)), dim3(64 * kKdaChunk), 0, st, a,
-                     blk);
-  int rc = mm::check_launch("kda_chunk prep");
+  // every token's channels 16-byte aligned: loads of 8 channels, else one by one
+  const bool f32 = a.g_dtype == MM_FP32;
+  const bool vec = mm::aligned16(a.q) && mm::aligned16(a.k) && mm::aligned16(a.g) && (!a.use_gate || mm::aligned16(a.dt_bias)) &&
+                   a.q_ts % 8 == 0 && a.k_ts % 8 == 0 && a.g_ts % (f32 ? 4 : 8) == 0;
+  int rc;
+  if (vec) rc = f32 ? launch_kda_prep<K, true, true>(a, ws, st) : launch_kda_prep<K, true, false>(a, ws, st);
+  else rc = f32 ? launch_kda_prep<K, false, true>(a, ws, st) : launch_kda_prep<K, false, false>(a, ws, st);
   if (rc) return rc;
-  constexpr int NWB = kKdaNwb, cols = NWB * kWave / (K / 4);
-  if (a.V % cols == 0) {
-    hipLaunchKernelGGL((kda_chunk_kernel<K, NWB>), dim3(static_cast<unsigned>(a.V / cols), static_cast<unsigned>(a.H)),
-                       dim3(kWave * NWB), 0, st, a, static_cast<const float*>(blk));
-  } else {  // V a multiple of 8 only: one wave per workgroup
-    hipLaunchKernelGGL((kda_chunk_kernel<K, 1>), dim3(static_cast<unsigned>(a.V / (cols / NWB)),
-                       static_cast<unsigned>(a.H)), dim3(kWave), 0, st, a, static_cast<const float*>(blk));
-  }
+  const dim3 grid(static_cast<unsigned>(a.H), static_cast<unsigned>((a.V + 15) / 16));
+  const bool far = a.v_ts >= (1 << 25) || a.o_ts >= (1 << 25);
+  auto kern = far ? kda_chunk_kernel<K, true> : kda_chunk_kernel<K, false>;
+  rc = mm::allow_lds(kern, KdaLds<K>::BYTES, "kda_chunk");
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, grid, dim3(320), KdaLds<K>::BYTES, st, a, static_cast<const float*>(ws));
   return mm::check_launch("kda_chunk");
 }
 

@@ -52,10 +52,11 @@ import thinker_attn as TA
 __all__ = ["FastThinkerStep"]
 
 _SCORING = ("sigmoid", "softmax")
-# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda), as the engine switches its KDA layers'
-# mode (engine.py:946-949, 964-967). Measured per call over 16 heads of 128 x 128 (graph replays): 200 / 256 / 384 /
-# 512 tokens 42.1 / 48.2 / 71.2 / 87.1 us chunked against 43.2 / 51.7 / 72.7 / 93.4 us recurrent.
-KDA_CHUNK_ABOVE = 192
+# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda); the engine switches its KDA layers' mode
+# past 192 (engine.py:946-949, 964-967), here both forms compute the same and the line lies where the chunked one is the
+# faster: us per layer's core at 16 / 32 / 64 / 150 / 192 rows 11.3 / 12.2 / 14.3 / 20.1 / 21.9 chunked, 10.8 / 13.9 /
+# 19.7 / 35.4 / 40.9 recurrent.
+KDA_CHUNK_ABOVE = 24
 
 
 def _norm(mod, what):
@@ -263,8 +264,8 @@ class FastThinkerStep:
         """The attention half of layer li over a prompt's T rows h [T, H] at positions pos_buf .. pos_buf + T - 1:
         h + o(mixer(input_layernorm(h))). KDA: the projection, the q / k / v short convolutions (their caches end
         on the prompt's last real inputs), the f / g LoRA up-projections, the recurrence from the layer's state
-        (fused_recurrent_kda up to KDA_CHUNK_ABOVE rows, chunk_kda beyond: the engine's mode switch,
-        engine.py:946-949; padding rows past n_valid leave the state unchanged), rms_norm_gated; MLA: the
+        (fused_recurrent_kda up to KDA_CHUNK_ABOVE rows, chunk_kda beyond; padding rows past n_valid leave the state
+        unchanged), rms_norm_gated; MLA: the
         q | k | v projection and mla_prefill_attn (padding rows are stored past the real ones, where the next
         decode steps overwrite them before any query reads them). own: h is the step's and dead after this call, so
         the o projection past fastlinear.MAX_M rows adds into it in place."""

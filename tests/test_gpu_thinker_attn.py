@@ -70,6 +70,50 @@ def test_kda_chunk_matches_oracle(T, H, K, V, gate):
     torch.testing.assert_close(fin[0].cpu().double(), rS, rtol=1e-3, atol=1e-4)
 
 
+@pytest.mark.parametrize("T,H,K,V,gdt,off", [
+    (15, 2, 128, 16, BF, 0), (17, 2, 128, 8, torch.float32, 0), (48, 1, 64, 24, BF, 1), (63, 3, 128, 40, BF, 1),
+    (64, 2, 64, 64, torch.float32, 1), (65, 9, 128, 128, BF, 0), (97, 2, 128, 136, torch.float32, 3)])
+def test_kda_chunk_groups_columns_and_alignment(T, H, K, V, gdt, off):
+    """Chunk counts around the four chunks in flight, column tiles that end inside, bf16 and fp32 gates, and rows that
+    start off a 16-byte boundary (loads one by one): outputs to bf16 and the state to fp32 sums, against float64."""
+    print(f"[kda chunk groups] T={T} H={H} K={K} V={V} {gdt} off={off}", flush=True)
+    q, k, v, g, beta, A_log, dt, S0 = _kda_inputs(T, H, K, V, 900 + T, gdt)
+
+    def shifted(x):
+        b = torch.empty(x.numel() + off, device=DEV, dtype=x.dtype)
+        return b[off:].view_as(x).copy_(x)
+    o, fin = TA.chunk_kda(shifted(q), shifted(k), shifted(v), shifted(g), beta, A_log=A_log, dt_bias=shifted(dt),
+                          initial_state=S0, output_final_state=True, use_qk_l2norm_in_kernel=True,
+                          use_gate_in_kernel=True)
+    ro, rS = A.kda_recurrent(q[0].cpu(), k[0].cpu(), v[0].cpu(), g[0].cpu(), beta[0].cpu(), S0[0].cpu(),
+                             A_log=A_log.cpu(), dt_bias=dt.cpu())
+    close(o[0], ro)
+    # fp32 sums of at most T + 128 terms of size 1: (T + 128) 2^-24 of the state's scale (0.3 .. 1)
+    torch.testing.assert_close(fin[0].cpu().double(), rS, rtol=1e-4, atol=(T + 128) * 2.0 ** -24)
+
+
+def test_kda_chunk_nan_padding_and_far_token_strides():
+    """NaN in the values of padding tokens reaches neither the real tokens' outputs nor the state; tokens 2^25 elements
+    apart (their own kernel) equal the same prompt packed, bit for bit."""
+    T, n, H, K, V = 40, 19, 2, 128, 128
+    q, k, v, g, beta, A_log, dt, S0 = _kda_inputs(T, H, K, V, 980)
+    v[:, n:] = float("nan")
+    kw = dict(A_log=A_log, dt_bias=dt, use_qk_l2norm_in_kernel=True, use_gate_in_kernel=True, output_final_state=True)
+    print("[kda chunk nan padding]", flush=True)
+    o, fin = TA.chunk_kda(q, k, v, g, beta, initial_state=S0, n_valid=torch.tensor([n], device=DEV), **kw)
+    o1, fin1 = TA.chunk_kda(q[:, :n], k[:, :n], v[:, :n], g[:, :n], beta[:, :n], initial_state=S0, **kw)
+    assert torch.equal(o[:, :n], o1) and torch.equal(fin, fin1) and torch.isfinite(fin).all()
+    T = 5
+    q, k, v, g, beta, A_log, dt, S0 = _kda_inputs(T, H, K, V, 990)
+    far = torch.zeros((T - 1) * 2 ** 25 + H * V, device=DEV, dtype=BF).as_strided((1, T, H, V), (0, 2 ** 25, V, 1))
+    far.copy_(v)
+    kw.update(A_log=A_log, dt_bias=dt)
+    print("[kda chunk far strides]", flush=True)
+    a, fa = TA.chunk_kda(q, k, v, g, beta, initial_state=S0, **kw)
+    b, fb = TA.chunk_kda(q, k, far, g, beta, initial_state=S0, **kw)
+    assert torch.equal(a, b) and torch.equal(fa, fb)
+
+
 def test_kda_chunk_full_prompt_and_strong_decay():
     """The hybrid thinker's shape, 512 tokens over 16 heads of 128 x 128, against the float64 recurrence; then decays
     of e^-30 .. e^-80 per token, whose products over a chunk underflow: the chunk form takes them as products, never
