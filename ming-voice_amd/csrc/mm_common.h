@@ -58,6 +58,7 @@ namespace mmd {
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 
@@ -156,6 +157,8 @@ constexpr int kDppXor1 = 0xB1;         // quad_perm [1,0,3,2]: lane i <-> i ^ 1
 constexpr int kDppXor2 = 0x4E;         // quad_perm [2,3,0,1]: lane i <-> i ^ 2
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7 - i within 8 lanes
 constexpr int kDppMirror = 0x140;      // lane i <-> 15 - i within 16 lanes
+constexpr int kDppRor4 = 0x124;        // lanes of 16 rotated by 4, by 8
+constexpr int kDppRor8 = 0x128;
 
 // Sum over aligned groups of `width` lanes (a power of two <= 64); every lane of a group gets the group's
 // total, with one fixed association: pairs, then quads, then halves and rows of 16 (each step adds a lane

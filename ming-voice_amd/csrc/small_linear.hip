@@ -1,5 +1,6 @@
 // Small-M linear, M <= 16 (fastlinear.py:123-174): y = act(norm?(x) . W^T + b) [+ residual].
-// HBM-bound GEMV, latency-bound at decode sizes (a few MB per call). For rows of up to 1024 16-byte chunks
+// HBM-bound GEMV, latency-bound at decode sizes (a few MB per call). Several rows of up to 4096 elements take the matrix
+// units (small_linear_rows_kernel, below); one row, and longer ones, the vector form. For rows of up to 1024 16-byte chunks
 // (K <= 8192) one pass covers the row: a wave shares each of its rows across its 64 lanes and issues all
 // weight loads of its rows at once, so it waits for memory once; the activation chunks come from the L1/L2
 // caches. The optional RMSNorm prologue is fused there: the lanes of a wave hold the whole activation row,
@@ -252,6 +253,190 @@ __global__ __launch_bounds__(256) void small_linear_1pass_kernel(LinArgs a, cons
   }
 }
 
+// ---------------------------------------------------------------------------------- several rows, matrix units
+//
+// M = 2 .. 16 rows: the dots of 4 weight rows with 4 token rows on v_mfma_f32_4x4x4_16b_bf16, whose 16 blocks take 16
+// different k groups of the same rows: lane 4 b + r gives 4 k of block b of weight row r and of token row r, and block b
+// of D holds its part of every (weight row, token row) pair (weight row in the register, token row r). So a weight chunk
+// is read once by one lane for all tokens, in 256-byte pieces of a row, and a pair costs 1/64 of an 8-cycle instruction
+// per 4 k where the vector form takes two dots per lane and an own sum over the lanes (6 rows: 12 sums of 6 steps).
+// A workgroup of 4 waves takes 4 RQ weight rows, each wave a quarter of k; the waves' totals meet in LDS.
+// us per launch (rows: K -> N, n with the norm fused), the vector form -> this one: 6: 1024 -> 3072 n 5.6 -> 4.2, 1024 ->
+// 1024 3.2 -> 2.5, 1024 -> 4096 n 6.3 -> 4.6, 4096 -> 1024 5.5 -> 4.6; 2: 1024 -> 3072 n 4.6 -> 3.4; 16: 2048 -> 6416 n
+// 26.2 -> 17.3, 2048 -> 2048 9.3 -> 5.4 (a launch alone is about 2).
+template <int NC, int TG, int RQ, bool NORM, bool GLU>
+__global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const uint16_t* __restrict__ norm_g,
+                                                                float norm_eps) {
+  static_assert(!GLU || RQ == 2, "GLU: a quad of gate rows and its quad of up rows");
+  constexpr int V = RQ * TG * 4;             // totals per lane group: (weight quad q, token group t, weight row) in order
+  constexpr int NR = GLU ? 4 : 4 * RQ;       // output columns of the workgroup
+  __shared__ float s_ss[4][TG * 4];
+  __shared__ float s_part[4][V][4];
+  const int lane = lane_id(), wave = threadIdx.x / kWave, b = lane >> 2, r = lane & 3;
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * NR;
+  const uint32_t nch = static_cast<uint32_t>(a.K / 8);
+  // every load of the lane first: its chunks of the weight rows, the token rows and the norm weights
+  uint4 wv[RQ][NC], xv[TG][NC], gv[NC];
+  const rsrc_t xr = make_rsrc(a.x, ((a.M - 1) * a.xs + a.K) * 2), gr = make_rsrc(norm_g, NORM ? a.K * 2 : 0);
+  uint32_t c16[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const uint32_t c = (wave * NC + j) * 16 + b;
+    c16[j] = c < nch ? c * 16u : kPast;
+  }
+#pragma unroll
+  for (int q = 0; q < RQ; ++q) {
+    const int64_t row = GLU ? n0 + q * a.N : n0 + 4 * q, left = GLU ? a.N - n0 : a.N - row;  // its rows: 4 at most
+    const rsrc_t wr = make_rsrc(a.w + (left > 0 ? row : 0) * a.ws, left > 0 ? ((min(left, static_cast<int64_t>(4)) - 1) * a.ws + a.K) * 2 : 0);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) wv[q][j] = buf16(wr, c16[j] == kPast ? kPast : static_cast<uint32_t>(r * a.ws) * 2u + c16[j]);
+  }
+#pragma unroll
+  for (int t = 0; t < TG; ++t)
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      xv[t][j] = buf16(xr, c16[j] == kPast || 4 * t + r >= a.M ? kPast : static_cast<uint32_t>((4 * t + r) * a.xs) * 2u + c16[j]);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) gv[j] = buf16(gr, c16[j]);
+  }
+  // this thread's output: token row em, column n0 + en
+  const int em = threadIdx.x / NR, en = threadIdx.x % NR;
+  const bool live = em < a.M && n0 + en < a.N;
+  const rsrc_t br = make_rsrc(a.b, !GLU && a.b ? a.N * 2 : 0);
+  const rsrc_t rr = make_rsrc(a.res, !GLU && a.res ? ((a.M - 1) * a.rs + a.N) * 2 : 0);
+  const float bias = bf16_to_f32(buf2(br, live ? static_cast<uint32_t>(n0 + en) * 2u : kPast));
+  const float res = bf16_to_f32(buf2(rr, live ? static_cast<uint32_t>(em * a.rs + n0 + en) * 2u : kPast));
+  if constexpr (NORM) {
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) ss += sumsq8(xv[t][j]);
+      ss += dpp_f32<kDppRor8>(ss);
+      ss += dpp_f32<kDppRor4>(ss);
+      ss = half_pair_sum(row_pair_sum(ss));
+      if (b == 0) s_ss[wave][4 * t + r] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+      const float tot = ((s_ss[0][4 * t + r] + s_ss[1][4 * t + r]) + s_ss[2][4 * t + r]) + s_ss[3][4 * t + r];
+      const float rstd = 1.0f / sqrtf(tot / static_cast<float>(a.K) + norm_eps);
+#pragma unroll
+      for (int j = 0; j < NC; ++j) xv[t][j] = norm_chunk(xv[t][j], gv[j], rstd, a.norm_once);
+    }
+  }
+  floatx4 acc[RQ][TG];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int t = 0; t < TG; ++t) acc[q][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < RQ; ++q)
+#pragma unroll
+        for (int t = 0; t < TG; ++t) {
+          const uint2 w2 = h ? make_uint2(wv[q][j].z, wv[q][j].w) : make_uint2(wv[q][j].x, wv[q][j].y);
+          const uint2 x2 = h ? make_uint2(xv[t][j].z, xv[t][j].w) : make_uint2(xv[t][j].x, xv[t][j].y);
+          acc[q][t] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4_t, w2), __builtin_bit_cast(s16x4_t, x2),
+                                                             acc[q][t], 0, 0, 0);
+        }
+  // the 16 blocks' parts: split between the wave's halves and row pairs (each keeps half of the values), then summed
+  // over the 4 blocks of a row
+  float x[V];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[(q * TG + t) * 4 + v] = acc[q][t][v];
+#pragma unroll
+  for (int v = 0; v < V / 2; ++v) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[v]), __float_as_uint(x[v + V / 2]), false, false);
+    x[v] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int v = 0; v < V / 4; ++v) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + V / 4]), false, false);
+    x[v] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+  const int first = (lane >> 5) * (V / 2) + ((lane >> 4) & 1) * (V / 4);
+#pragma unroll
+  for (int v = 0; v < V / 4; ++v) {
+    x[v] += dpp_f32<kDppRor8>(x[v]);
+    x[v] += dpp_f32<kDppRor4>(x[v]);
+    if ((lane & 12) == 0) s_part[wave][first + v][r] = x[v];
+  }
+  __syncthreads();
+  if (!live) return;
+  auto total = [&](int q, int row) {
+    const int v = (q * TG + em / 4) * 4 + row;
+    return ((s_part[0][v][em % 4] + s_part[1][v][em % 4]) + s_part[2][v][em % 4]) + s_part[3][v][em % 4];
+  };
+  uint16_t* y = a.y + em * a.ys + n0 + en;
+  if constexpr (GLU) {
+    *y = f32_to_bf16(round_bf16(silu(round_bf16(total(0, en)))) * round_bf16(total(1, en)));
+  } else {
+    const float keep = total(en / 4, en % 4);
+    float v = apply_act(a.b ? keep + bias : keep, a.act);
+    if (a.res) v = round_bf16(v) + res;
+    *y = f32_to_bf16(v);
+  }
+}
+
+template <int NC, int TG, int RQ, bool GLU>
+int launch_rows_rq(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
+  constexpr int NR = GLU ? 4 : 4 * RQ;
+  const dim3 grid(static_cast<unsigned>((a.N + NR - 1) / NR));
+  if (g) hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, true, GLU>), grid, dim3(256), 0, st, a, g, eps);
+  else hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, false, GLU>), grid, dim3(256), 0, st, a, g, eps);
+  return mm::check_launch(GLU ? "small_linear_glu" : "small_linear");
+}
+
+// Weight rows per workgroup: more of them read the token rows less often, fewer give more workgroups. us at 4 | 8 | 16
+// rows: N = 4096, 6 rows of 1024 6.4 | 5.3 | 4.6; 3072 5.2 | 4.8 | 4.2; 2048, 16 rows of 2048 6.8 | 5.4 | 6.2; 1152, 3
+// rows of 896 3.2 | 2.9 | 3.3; 1024, 6 rows of 1024 2.5 | 2.7 | 3.3, of 4096 4.6 | 5.4 | 7.1.
+template <int NC, int TG, bool GLU>
+int launch_rows_tg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
+  if constexpr (GLU) {
+    return launch_rows_rq<NC, TG, 2, true>(a, g, eps, st);
+  } else {
+    const int64_t cus = mm::cu_count();
+    if constexpr (NC <= 4) {
+      if (a.N >= 12 * cus) return launch_rows_rq<NC, TG, 4, false>(a, g, eps, st);
+    }
+    if (a.N > 4 * cus) return launch_rows_rq<NC, TG, 2, false>(a, g, eps, st);
+    return launch_rows_rq<NC, TG, 1, false>(a, g, eps, st);
+  }
+}
+
+template <int NC, bool GLU>
+int launch_rows_nc(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
+  if (a.M <= 4) return launch_rows_tg<NC, 1, GLU>(a, g, eps, st);
+  if (a.M <= 8) return launch_rows_tg<NC, 2, GLU>(a, g, eps, st);
+  if constexpr (NC <= 4) return launch_rows_tg<NC, 4, GLU>(a, g, eps, st);
+  return MM_ERR_ARG;
+}
+
+// Whether the matrix-unit form takes (M, K): its lanes hold all their chunks of the token rows at once, and a row group
+// and the tokens are addressed by 32-bit offsets.
+bool rows_form(const LinArgs& a) {
+  if (a.M < 2 || a.K > 4096 || (a.M > 8 && a.K > 2048)) return false;
+  return a.ws < (1LL << 27) && mm::rsrc_fits((static_cast<int64_t>(a.M) * a.xs + a.K) * 2);
+}
+
+template <bool GLU>
+int launch_rows(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
+  if (a.K <= 512) return launch_rows_nc<1, GLU>(a, g, eps, st);
+  if (a.K <= 1024) return launch_rows_nc<2, GLU>(a, g, eps, st);
+  if (a.K <= 2048) return launch_rows_nc<4, GLU>(a, g, eps, st);
+  return launch_rows_nc<8, GLU>(a, g, eps, st);
+}
+
 // Rows longer than one pass: each wave computes GPW = 64/LPR rows at a time, R times; LPR lanes share one
 // row, NC chunks per lane per pass.
 template <int LPR, int NC, int R>
@@ -370,6 +555,7 @@ extern "C" int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_ro
               static_cast<const uint16_t*>(b), act, once, static_cast<const uint16_t*>(residual), res_row_stride,
               static_cast<uint16_t*>(y), y_row_stride};
     auto g = static_cast<const uint16_t*>(norm_g);
+    if (rows_form(a)) return launch_rows<false>(a, g, norm_eps, st);
     // chunks per lane NC = ceil(nch / 64), rounded up to an instantiated size; at most 16 loads per lane
     // (rows per wave measured on MI355X: 2 at K = 896; at K = 2048 1 up to N = 2048, 2 from N = 16 per CU on,
     // where each wave's activation row (and norm weights) from L2 then serves two weight rows: one token,
@@ -426,6 +612,7 @@ extern "C" int mm_small_linear_glu(const void* x, int64_t M, int64_t K, int64_t 
             inter, w_row_stride, nullptr, MM_ACT_NONE, false, nullptr, 0, static_cast<uint16_t*>(y), y_row_stride};
   auto g = static_cast<const uint16_t*>(norm_g);
   hipStream_t st = MM_STREAM(stream);
+  if (rows_form(a)) return launch_rows<true>(a, g, norm_eps, st);
   const int64_t nch = K / 8;
   if (nch <= 64) return launch_glu<1>(a, g, norm_eps, st);
   if (nch <= 128) return launch_glu<2>(a, g, norm_eps, st);

@@ -27,23 +27,38 @@ __global__ __launch_bounds__(64) void rope_attn_kernel(const uint16_t* __restric
   const int lane = lane_id();
   const int b = blockIdx.x / H, h = blockIdx.x % H;
   const int P = HD / 2;
+  // every load first, rows and dims past the ends clamped to the last (a load behind its own range test is waited on
+  // before the next is issued)
+  uint16_t qr[SP][NT], kr[SP][NT], vr[SP][NT];
+  float c[SP][NT], si[SP][NT];
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    const int sl = min(s, S - 1);
+    const uint16_t* row = qkv + (static_cast<int64_t>(b) * S + sl) * 3 * D + static_cast<int64_t>(h) * HD;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int d = min(lane + 64 * t, HD - 1);
+      qr[s][t] = row[d];
+      kr[s][t] = row[D + d];
+      vr[s][t] = row[2 * D + d];
+      c[s][t] = cs[sl * P + (d >> 1)];
+      si[s][t] = sn[sl * P + (d >> 1)];
+    }
+  }
   float q2[SP][NT], k2[SP][NT], v[SP][NT];
 #pragma unroll
   for (int s = 0; s < SP; ++s) {
-    const uint16_t* row = qkv + (static_cast<int64_t>(b) * S + s) * 3 * D + static_cast<int64_t>(h) * HD;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int d = lane + 64 * t;
       const bool ok = s < S && d < HD;
-      const float q = ok ? bf16_to_f32(row[d]) : 0.f;
-      const float k = ok ? bf16_to_f32(row[D + d]) : 0.f;
-      v[s][t] = ok ? bf16_to_f32(row[2 * D + d]) : 0.f;
-      const float c = ok ? cs[s * P + (d >> 1)] : 1.f;
-      const float si = ok ? sn[s * P + (d >> 1)] : 0.f;
+      const float q = ok ? bf16_to_f32(qr[s][t]) : 0.f;
+      const float k = ok ? bf16_to_f32(kr[s][t]) : 0.f;
+      v[s][t] = ok ? bf16_to_f32(vr[s][t]) : 0.f;
       const float qp = __shfl_xor(q, 1, kWave), kp = __shfl_xor(k, 1, kWave);
-      const float sg = (d & 1) ? si : -si;  // even: x cos - partner sin; odd: x cos + partner sin
-      q2[s][t] = round_bf16(fmaf(qp, sg, q * c));
-      k2[s][t] = round_bf16(fmaf(kp, sg, k * c));
+      const float sg = (d & 1) ? si[s][t] : -si[s][t];  // even: x cos - partner sin; odd: x cos + partner sin
+      q2[s][t] = round_bf16(fmaf(qp, sg, q * c[s][t]));
+      k2[s][t] = round_bf16(fmaf(kp, sg, k * c[s][t]));
     }
   }
   float o[SP][NT];

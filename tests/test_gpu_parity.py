@@ -717,6 +717,36 @@ def test_small_linear(M, KN):
     close(y, O.small_linear(x.cpu(), w.cpu(), norm=(g.cpu(), 1e-6)))
 
 
+@pytest.mark.parametrize("M,K,N", [(2, 8, 1), (3, 504, 5), (4, 512, 1023), (5, 520, 1029), (8, 1016, 3073), (9, 1024, 3075),
+                                   (16, 2048, 2051), (8, 2056, 1026), (8, 4096, 1029), (9, 2056, 9), (8, 4104, 9)])
+def test_small_linear_rows_edges(M, K, N):
+    """Several rows on the matrix units: token groups of 4, weight rows 4, 8 and 16 to a workgroup with a remainder, k
+    chunks that end inside a wave's share, and the first shapes past it; bias, activation, residual, norm (both
+    roundings), rows with a stride or repeated, and the gated pair, which equals the two projections bit for bit. Sums of
+    K products in fp32: K 2^-24 of the sum of the magnitudes, and the bf16 rounding of the result."""
+    print(f"[small_linear rows] M={M} K={K} N={N}", flush=True)
+    x = W.normal((M, K + 8), 1.0, 130 + M, DEV)[:, :K]  # strided rows
+    w = W.normal((N, K), 0.05, 131, DEV)
+    b, r = W.normal((N,), 1.0, 132, DEV), W.normal((M, N), 1.0, 133, DEV)
+    g = W.normal((K,), 0.02, 134, DEV, mean=1.0)
+
+    def near(y, xin):
+        want = xin.double() @ w.double().t()
+        mag = xin.double().abs() @ w.double().abs().t()
+        bound = (K + 8) * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs() + 1e-30
+        assert ((y.double() - want).abs() <= bound).all()
+    near(fastlinear.small_linear(x, w), x)
+    one = x[:1].expand(M, -1)  # the same row M times: stride 0
+    near(fastlinear.small_linear(one, w), one)
+    y = fastlinear.small_linear(x, w, b, act=1, residual=r, norm=(g, 1e-6))
+    close(y, O.small_linear(x.cpu(), w.cpu(), b.cpu(), 1, r.cpu(), norm=(g.cpu(), 1e-6)))
+    if N % 2 == 1:
+        wgu = W.normal((2 * N, K), 0.05, 135, DEV)
+        import fast_talker as FT
+        assert torch.equal(FT.gate_up_silu(x, wgu, norm=(g, 1e-6)),
+                           FT.silu_mul(fastlinear.small_linear(x, wgu, norm=(g, 1e-6))))
+
+
 def test_small_linear_lm_head_shape():
     x = W.normal((1, 2048), 1.0, 110, DEV)
     w = W.normal((126464, 2048), 0.02, 111, DEV)
