@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void decode_attn_split_kernel(AttnArgs a) {
   __shared__ __align__(16) float ls[kAttnMaxHd / 2];
   __shared__ __align__(16) float lp[kWaves][kTile * kMaxGroup];  // p[position][head] per wave
   __shared__ float lm[kWaves][kMaxGroup], ll[kWaves][kMaxGroup];
-  __shared__ __align__(16) float lacc[kWaves - 1][GP * 64 * NDV];  // waves 1..3: acc[head][d]
+  __shared__ __align__(16) float lacc[kWaves][GP * 64 * NDV];  // acc[head][d]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int c = blockIdx.x, kvh = blockIdx.y;
   const int hd = a.hd, half = hd / 2, ks_n = hd / 32, G = a.nh / a.nkv;
@@ -301,18 +301,17 @@ __global__ __launch_bounds__(256) void decode_attn_split_kernel(AttnArgs a) {
         for (int j = 0; j < NDV; ++j) acc[4 * g4 + u][j] = fmaf(pg[u], vt[j], acc[4 * g4 + u][j]);
     }
   }
-  if (wave > 0) {
 #pragma unroll
-    for (int g = 0; g < GP; ++g)
+  for (int g = 0; g < GP; ++g)
 #pragma unroll
-      for (int j = 0; j < NDV; ++j) lacc[wave - 1][g * 64 * NDV + lane + 64 * j] = acc[g][j];
-  }
+    for (int j = 0; j < NDV; ++j) lacc[wave][g * 64 * NDV + lane + 64 * j] = acc[g][j];
   __syncthreads();
-  if (wave != 0) return;
-  // wave 0 holds position c0 <= pos, so its max is finite and so is the chunk's
+  // the chunk's (m, l, acc): wave w merges the heads w, w + 4, ... (wave 0 holds position c0 <= pos, so its max is finite
+  // and so is the chunk's)
   const int64_t hbase = static_cast<int64_t>(kvh) * G;
 #pragma unroll
-  for (int g = 0; g < GP; ++g) {
+  for (int gg = 0; gg < G4; ++gg) {
+    const int g = 4 * gg + wave;
     const float m = fmaxf(fmaxf(lm[0][g], lm[1][g]), fmaxf(lm[2][g], lm[3][g]));
     float w[kWaves];
 #pragma unroll
@@ -320,9 +319,9 @@ __global__ __launch_bounds__(256) void decode_attn_split_kernel(AttnArgs a) {
     float s[NDV];
 #pragma unroll
     for (int j = 0; j < NDV; ++j) {
-      s[j] = acc[g][j] * w[0];
+      s[j] = lacc[0][g * 64 * NDV + lane + 64 * j] * w[0];
 #pragma unroll
-      for (int wv = 1; wv < kWaves; ++wv) s[j] = fmaf(lacc[wv - 1][g * 64 * NDV + lane + 64 * j], w[wv], s[j]);
+      for (int wv = 1; wv < kWaves; ++wv) s[j] = fmaf(lacc[wv][g * 64 * NDV + lane + 64 * j], w[wv], s[j]);
     }
     if (g < G) {
       float* dst = a.ws_acc + ((hbase + g) * a.nc + c) * hd;
