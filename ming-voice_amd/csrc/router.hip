@@ -121,25 +121,29 @@ __global__ __launch_bounds__(256) void router_gemv_kernel(const typename TX::T* 
 }
 
 // The same for bf16 rows of at most 2048 * J elements (H a multiple of 8, 16-byte aligned rows), in one
-// memory round trip: thread i owns the 8-element chunks i + 256 j, and every load of the workgroup (its
-// router row, the RMSNorm weight, the token rows) is issued at kernel start through buffer resources.
-// The sum of squares runs over the chunks exactly as row_rstd256 does, so xn matches mm_rms_norm bit for
-// bit; a chunk's logit terms are added in element order, chunks in j order, then the waves in order.
-template <int J, int NT>
-__global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* __restrict__ x, int n_tokens, int64_t H,
-                                                               int64_t xs, const float* __restrict__ w32, int E,
+// memory round trip, a workgroup per expert and token (grid (E, tokens)): thread i owns the 8-element chunks
+// i + 256 j, and every load of the workgroup (its router row, the RMSNorm weight, the token row) is issued at
+// kernel start through buffer resources. The sum of squares runs over the chunks exactly as row_rstd256 does, so
+// xn matches mm_rms_norm bit for bit; a chunk's logit terms are added in element order, chunks in j order, then
+// the waves in order. Bound by its chain (load, norm, dot), so every token takes its own workgroup, the router
+// rows coming from cache: a decode block of 5 / 7 tokens 22.0 / 25.2 us with 8 tokens to a workgroup, 20.5 / 22.9
+// with 2, 20.1 / 22.5 with one (64 experts of a tiny inner size, so that the front is what counts).
+template <int J>
+__global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* __restrict__ x, int64_t H, int64_t xs,
+                                                               const float* __restrict__ w32, int E,
                                                                float* __restrict__ logits,
                                                                const uint16_t* __restrict__ norm_w, float eps,
                                                                uint16_t* __restrict__ xn_out) {
-  __shared__ float red_ss[NT][4];
-  __shared__ float red[4][NT];
+  __shared__ float red_ss[4];
+  __shared__ float red[4];
   const int e = blockIdx.x;
+  const int64_t t = blockIdx.y;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   const int nch = static_cast<int>(H / 8);
   const rsrc_t wr = make_rsrc(w32 + static_cast<int64_t>(e) * H, H * 4);
-  const rsrc_t xr = make_rsrc(x, static_cast<int64_t>(n_tokens) * xs * 2);
+  const rsrc_t xr = make_rsrc(x + t * xs, H * 2);
   const rsrc_t nr = make_rsrc(norm_w, norm_w ? H * 2 : 0);
-  uint4 wv[J][2], nv[J], xv[J][NT];
+  uint4 wv[J][2], nv[J], xv[J];
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int c = tid + 256 * j;
@@ -147,69 +151,44 @@ __global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* _
     wv[j][0] = buf16(wr, ok ? static_cast<uint32_t>(c) * 32u : kPast);
     wv[j][1] = buf16(wr, ok ? static_cast<uint32_t>(c) * 32u + 16u : kPast);
     nv[j] = buf16(nr, ok ? static_cast<uint32_t>(c) * 16u : kPast);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)  // a token past n_tokens reads zero (no branch: a load behind one is waited on)
-      xv[j][t] = buf16(xr, ok && t < n_tokens ? static_cast<uint32_t>(t * xs * 2 + c * 16) : kPast);
+    xv[j] = buf16(xr, ok ? static_cast<uint32_t>(c) * 16u : kPast);
   }
-  float rstd[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) rstd[t] = 1.f;
+  float rstd = 1.f;
   if (norm_w) {
+    float ss = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (t < n_tokens) {
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < J; ++j) ss = chunk_ss_bf16x8(xv[j][t], ss);
-        ss = wave_sum(ss);
-        if (lane == 0) red_ss[t][wave] = ss;
-      }
-    }
+    for (int j = 0; j < J; ++j) ss = chunk_ss_bf16x8(xv[j], ss);
+    ss = wave_sum(ss);
+    if (lane == 0) red_ss[wave] = ss;
     __syncthreads();
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      if (t < n_tokens)
-        rstd[t] = rsqrtf((((red_ss[t][0] + red_ss[t][1]) + red_ss[t][2]) + red_ss[t][3]) / static_cast<float>(H) + eps);
+    rstd = rsqrtf((((red_ss[0] + red_ss[1]) + red_ss[2]) + red_ss[3]) / static_cast<float>(H) + eps);
   }
   const bool store_xn = xn_out && e == 0;
-  float acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = 0.f;
+  float acc = 0.f;
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int c = tid + 256 * j;
     const uint32_t wq[8] = {wv[j][0].x, wv[j][0].y, wv[j][0].z, wv[j][0].w, wv[j][1].x, wv[j][1].y, wv[j][1].z, wv[j][1].w};
     const uint32_t nq[4] = {nv[j].x, nv[j].y, nv[j].z, nv[j].w};
+    const uint32_t xq[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+    uint32_t o[4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (t < n_tokens) {
-        const uint32_t xq[4] = {xv[j][t].x, xv[j][t].y, xv[j][t].z, xv[j][t].w};
-        uint32_t o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float lo = __uint_as_float(xq[i] << 16), hi = __uint_as_float(xq[i] & 0xffff0000u);
-          if (norm_w) {
-            lo = round_bf16(__uint_as_float(nq[i] << 16) * round_bf16(lo * rstd[t]));
-            hi = round_bf16(__uint_as_float(nq[i] & 0xffff0000u) * round_bf16(hi * rstd[t]));
-          }
-          o[i] = static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
-          acc[t] = fmaf(lo, __uint_as_float(wq[2 * i]), acc[t]);
-          acc[t] = fmaf(hi, __uint_as_float(wq[2 * i + 1]), acc[t]);
-        }
-        if (store_xn && c < nch) reinterpret_cast<uint4*>(xn_out + t * H)[c] = make_uint4(o[0], o[1], o[2], o[3]);
+    for (int i = 0; i < 4; ++i) {
+      float lo = __uint_as_float(xq[i] << 16), hi = __uint_as_float(xq[i] & 0xffff0000u);
+      if (norm_w) {
+        lo = round_bf16(__uint_as_float(nq[i] << 16) * round_bf16(lo * rstd));
+        hi = round_bf16(__uint_as_float(nq[i] & 0xffff0000u) * round_bf16(hi * rstd));
       }
+      o[i] = static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
+      acc = fmaf(lo, __uint_as_float(wq[2 * i]), acc);
+      acc = fmaf(hi, __uint_as_float(wq[2 * i + 1]), acc);
     }
+    if (store_xn && c < nch) reinterpret_cast<uint4*>(xn_out + t * H)[c] = make_uint4(o[0], o[1], o[2], o[3]);
   }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < n_tokens) {
-      const float v = wave_sum(acc[t]);
-      if (lane == 0) red[wave][t] = v;
-    }
-  }
+  acc = wave_sum(acc);
+  if (lane == 0) red[wave] = acc;
   __syncthreads();
-  if (tid < n_tokens)
-    logits[static_cast<int64_t>(tid) * E + e] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+  if (tid == 0) logits[t * E + e] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // logits for many tokens on fp32 MFMA (v_mfma_f32_16x16x4_f32): a workgroup of 16 waves computes 16
@@ -440,6 +419,12 @@ int launch_select(const float* logits, int64_t n_tokens, int64_t E, const float*
   return mm::check_launch("router_select");
 }
 
+// Whether bf16 tokens take a workgroup per expert and token (router_gemv_bf16_kernel) rather than the MFMA tiles: up to
+// 8 tokens, and while that gives a CU at most 20 of them. us per prefill block of a tiny inner size, tiles | workgroups:
+// 64 experts, 9 / 16 / 37 / 64 / 100 / 150 tokens 46.4 | 40.7, 47.7 | 42.0, 49.4 | 45.0, 50.6 | 47.3, 51.1 | 49.8, 52.7 |
+// 53.7; 128 experts, 16 / 37 / 64 tokens 46.5 | 42.4, 47.4 | 45.6, 48.4 | 49.0.
+bool gemv_tokens(int64_t n_tokens, int64_t E) { return n_tokens <= 8 || n_tokens * E <= static_cast<int64_t>(20) * mm::cu_count(); }
+
 template <class TX>
 int launch_logits(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const float* w32, int64_t E, float* logits,
                   hipStream_t s, const void* norm_w = nullptr, float eps = 0.f, void* xn_out = nullptr) {
@@ -449,18 +434,12 @@ int launch_logits(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const 
   const bool fast = TX::kBf16 && (H & 7) == 0 && H <= 4096 && (xs & 7) == 0 && mm::aligned16(x) && mm::aligned16(w32) &&
                     (!norm_w || mm::aligned16(norm_w)) && (!xn_out || mm::aligned16(xn_out)) &&
                     n_tokens * xs * 2 < (1LL << 31);
-  if (n_tokens <= 8 && fast) {  // the RMSNorm is fused only for up to 8 tokens; larger batches take normalised rows
+  if (fast && gemv_tokens(n_tokens, E)) {
     const auto* xb = static_cast<const uint16_t*>(x);
-    const dim3 grid(static_cast<unsigned>(E));
-    const int nt = static_cast<int>(n_tokens), e = static_cast<int>(E);
-    if (H <= 2048 && n_tokens == 1)
-      hipLaunchKernelGGL((router_gemv_bf16_kernel<1, 1>), grid, dim3(256), 0, s, xb, nt, H, xs, w32, e, logits, nw, eps, xo);
-    else if (H <= 2048)
-      hipLaunchKernelGGL((router_gemv_bf16_kernel<1, 8>), grid, dim3(256), 0, s, xb, nt, H, xs, w32, e, logits, nw, eps, xo);
-    else if (n_tokens == 1)
-      hipLaunchKernelGGL((router_gemv_bf16_kernel<2, 1>), grid, dim3(256), 0, s, xb, nt, H, xs, w32, e, logits, nw, eps, xo);
-    else
-      hipLaunchKernelGGL((router_gemv_bf16_kernel<2, 8>), grid, dim3(256), 0, s, xb, nt, H, xs, w32, e, logits, nw, eps, xo);
+    const dim3 grid(static_cast<unsigned>(E), static_cast<unsigned>(n_tokens));
+    const int e = static_cast<int>(E);
+    if (H <= 2048) hipLaunchKernelGGL(router_gemv_bf16_kernel<1>, grid, dim3(256), 0, s, xb, H, xs, w32, e, logits, nw, eps, xo);
+    else hipLaunchKernelGGL(router_gemv_bf16_kernel<2>, grid, dim3(256), 0, s, xb, H, xs, w32, e, logits, nw, eps, xo);
   } else if (n_tokens <= 8) {
     hipLaunchKernelGGL(router_gemv_kernel<TX>, dim3(static_cast<unsigned>(E)), dim3(256), 0, s, xp,
                        static_cast<int>(n_tokens), H, xs, w32, static_cast<int>(E), logits, nw, eps, xo);
@@ -478,8 +457,8 @@ namespace mm {
 
 // Router of the MoE block front for bf16 tokens: RMSNorm (norm_w bf16, eps) into xn_out ([n_tokens, H]
 // bf16), logits of the normalised rows, then the selection with the shared expert appended. The norm runs
-// inside the logits kernel (router_gemv_bf16_kernel up to 8 tokens, router_norm_mfma_kernel above, each
-// workgroup normalising its 16 token rows); rows too long or misaligned for those normalise first
+// inside the logits kernel (router_gemv_bf16_kernel for few tokens, router_norm_mfma_kernel above, each
+// workgroup normalising its token rows); rows too long or misaligned for those normalise first
 // (mm_rms_norm). Either way xn is bit-identical. with_select false stops after the logits (a caller that
 // selects inside its next kernel).
 int router_front(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const void* norm_w, float eps,
@@ -489,7 +468,7 @@ int router_front(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const v
   int rc;
   const bool fused = n_tokens > 8 && H % 8 == 0 && H <= 4096 && xs % 8 == 0 && xn_out && aligned16(x) &&
                      aligned16(norm_w) && aligned16(xn_out) && aligned16(w32) && n_tokens * xs * 2 < (1LL << 31);
-  if (n_tokens <= 8) {
+  if (n_tokens <= 8 || (fused && gemv_tokens(n_tokens, sp.E))) {
     rc = launch_logits<BF16>(x, n_tokens, H, xs, w32, sp.E, logits, s, norm_w, eps, xn_out);
   } else if (fused) {  // the norm inside the logits kernel: one launch fewer
     dim3 grid(static_cast<unsigned>((sp.E + 15) / 16), static_cast<unsigned>((n_tokens + 15) / 16));

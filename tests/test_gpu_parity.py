@@ -754,6 +754,21 @@ def test_small_linear_lm_head_shape():
     close(y, O.small_linear(x.cpu(), w.cpu()))
 
 
+@pytest.mark.parametrize("H,E,n", [(2048, 64, 9), (2048, 64, 80), (2048, 64, 81), (1536, 128, 40), (1536, 128, 41),
+                                   (4096, 32, 30), (2056, 8, 33), (2048, 256, 21)])
+def test_router_logits_on_both_sides_of_the_tile_rule(H, E, n):
+    """The logits of few tokens (a workgroup per expert and token) and of more (MFMA tiles): against float64, sums of H
+    products in fp32 (H 2^-24 of the sum of the magnitudes at the most)."""
+    print(f"[router rule] H={H} E={E} n={n}", flush=True)
+    x, w32 = W.normal((n, H), 1.0, 140, DEV), W.normal((E, H), 0.02, 141, DEV, dtype=torch.float32)
+    g = W.normal((H,), 0.02, 142, DEV, mean=1.0)
+    xn = fused_ops.rms_norm(x, g, 1e-6)
+    logits = fused_ops.route(xn, w32, None, top_k=4, scoring="softmax")[2]
+    want = xn.double() @ w32.double().t()
+    bound = H * 2.0 ** -24 * (xn.double().abs() @ w32.double().abs().t())
+    assert ((logits.double() - want).abs() <= bound).all()
+
+
 # --------------------------------------------------------------------------------------------- hipGraph
 
 def test_decode_step_graph_replays_match_eager(blk):
