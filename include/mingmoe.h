@@ -55,6 +55,7 @@ extern "C" {
 /* ORed into small_linear's act: the norm prologue rounds once, bf16(x * rstd * g), as torch's F.rms_norm does on
  * the reference's path for more than 16 rows (fastlinear.py:151-160), instead of bf16(bf16(x * rstd) * g). */
 #define MM_NORM_ROUND_ONCE 0x100
+#define MM_ROW_INVARIANT 0x200
 
 /* Stacked expert weights, as the thinker lays them out (engine.py:150-188, 313-391):
  *   w_gu [n_slots, 2*inter, hidden]  rows 0..inter-1 = gate, inter..2*inter-1 = up
@@ -224,7 +225,8 @@ int mm_moe_block_prefill(const void* x, int64_t n_tokens, int64_t x_row_stride, 
  * x, w, b, residual, norm_g, y: bf16. norm_g (optional): RMSNorm prologue with norm_eps,
  * x -> bf16(bf16(x * rstd) * g), or bf16(x * rstd * g) with MM_NORM_ROUND_ONCE in act (the rounding of the
  * reference's torch path for M > 16, which callers run as 16-row pieces). b, residual, norm_g may be NULL.
- * act: MM_ACT_* (| MM_NORM_ROUND_ONCE).
+ * act: MM_ACT_* (| MM_NORM_ROUND_ONCE | MM_ROW_INVARIANT: every row gets the bits it gets with M = 1, whatever rows
+ * come with it; without it several rows may take the matrix units, whose sums run in another order).
  * xn_buf: bf16 scratch [M, K], used only when a norm prologue is given and K > 8192 (may be NULL otherwise);
  * shorter rows get the norm fused into the GEMV. x_row_stride 0 repeats one activation row M times. */
 int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_row_stride,

@@ -419,12 +419,6 @@ int launch_select(const float* logits, int64_t n_tokens, int64_t E, const float*
   return mm::check_launch("router_select");
 }
 
-// Whether bf16 tokens take a workgroup per expert and token (router_gemv_bf16_kernel) rather than the MFMA tiles: up to
-// 8 tokens, and while that gives a CU at most 20 of them. us per prefill block of a tiny inner size, tiles | workgroups:
-// 64 experts, 9 / 16 / 37 / 64 / 100 / 150 tokens 46.4 | 40.7, 47.7 | 42.0, 49.4 | 45.0, 50.6 | 47.3, 51.1 | 49.8, 52.7 |
-// 53.7; 128 experts, 16 / 37 / 64 tokens 46.5 | 42.4, 47.4 | 45.6, 48.4 | 49.0.
-bool gemv_tokens(int64_t n_tokens, int64_t E) { return n_tokens <= 8 || n_tokens * E <= static_cast<int64_t>(20) * mm::cu_count(); }
-
 template <class TX>
 int launch_logits(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const float* w32, int64_t E, float* logits,
                   hipStream_t s, const void* norm_w = nullptr, float eps = 0.f, void* xn_out = nullptr) {
@@ -434,7 +428,7 @@ int launch_logits(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const 
   const bool fast = TX::kBf16 && (H & 7) == 0 && H <= 4096 && (xs & 7) == 0 && mm::aligned16(x) && mm::aligned16(w32) &&
                     (!norm_w || mm::aligned16(norm_w)) && (!xn_out || mm::aligned16(xn_out)) &&
                     n_tokens * xs * 2 < (1LL << 31);
-  if (fast && gemv_tokens(n_tokens, E)) {
+  if (fast && n_tokens <= 8) {  // larger batches take the MFMA tiles, on normalised rows
     const auto* xb = static_cast<const uint16_t*>(x);
     const dim3 grid(static_cast<unsigned>(E), static_cast<unsigned>(n_tokens));
     const int e = static_cast<int>(E);
@@ -457,7 +451,7 @@ namespace mm {
 
 // Router of the MoE block front for bf16 tokens: RMSNorm (norm_w bf16, eps) into xn_out ([n_tokens, H]
 // bf16), logits of the normalised rows, then the selection with the shared expert appended. The norm runs
-// inside the logits kernel (router_gemv_bf16_kernel for few tokens, router_norm_mfma_kernel above, each
+// inside the logits kernel (router_gemv_bf16_kernel up to 8 tokens, router_norm_mfma_kernel above, each
 // workgroup normalising its token rows); rows too long or misaligned for those normalise first
 // (mm_rms_norm). Either way xn is bit-identical. with_select false stops after the logits (a caller that
 // selects inside its next kernel).
@@ -468,7 +462,7 @@ int router_front(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const v
   int rc;
   const bool fused = n_tokens > 8 && H % 8 == 0 && H <= 4096 && xs % 8 == 0 && xn_out && aligned16(x) &&
                      aligned16(norm_w) && aligned16(xn_out) && aligned16(w32) && n_tokens * xs * 2 < (1LL << 31);
-  if (n_tokens <= 8 || (fused && gemv_tokens(n_tokens, sp.E))) {
+  if (n_tokens <= 8) {
     rc = launch_logits<BF16>(x, n_tokens, H, xs, w32, sp.E, logits, s, norm_w, eps, xn_out);
   } else if (fused) {  // the norm inside the logits kernel: one launch fewer
     dim3 grid(static_cast<unsigned>((sp.E + 15) / 16), static_cast<unsigned>((n_tokens + 15) / 16));

@@ -1,6 +1,7 @@
 // Small-M linear, M <= 16 (fastlinear.py:123-174): y = act(norm?(x) . W^T + b) [+ residual].
 // HBM-bound GEMV, latency-bound at decode sizes (a few MB per call). Several rows of up to 4096 elements take the matrix
-// units (small_linear_rows_kernel, below); one row, and longer ones, the vector form. For rows of up to 1024 16-byte chunks
+// units (small_linear_rows_kernel, below) unless each is to get the bits it gets alone (MM_ROW_INVARIANT: the thinker's
+// short prompts); one row, and longer ones, the vector form. For rows of up to 1024 16-byte chunks
 // (K <= 8192) one pass covers the row: a wave shares each of its rows across its 64 lanes and issues all
 // weight loads of its rows at once, so it waits for memory once; the activation chunks come from the L1/L2
 // caches. The optional RMSNorm prologue is fused there: the lanes of a wave hold the whole activation row,
@@ -536,7 +537,8 @@ extern "C" int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_ro
   MM_REQUIRE(N <= 0x7fffffffLL * 8, "small_linear: N too large");
   MM_REQUIRE(x && w && y, "small_linear: null pointer");
   const bool once = (act & MM_NORM_ROUND_ONCE) != 0;
-  act &= ~MM_NORM_ROUND_ONCE;
+  const bool invariant = (act & MM_ROW_INVARIANT) != 0;
+  act &= ~(MM_NORM_ROUND_ONCE | MM_ROW_INVARIANT);
   MM_REQUIRE(act == MM_ACT_NONE || act == MM_ACT_GELU_TANH || act == MM_ACT_SILU, "small_linear: unknown act %d", act);
   MM_REQUIRE((x_row_stride >= K || x_row_stride == 0) && w_row_stride >= K && y_row_stride >= N,
              "small_linear: row stride too small (x rows may also repeat one row, stride 0)");
@@ -555,7 +557,7 @@ extern "C" int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_ro
               static_cast<const uint16_t*>(b), act, once, static_cast<const uint16_t*>(residual), res_row_stride,
               static_cast<uint16_t*>(y), y_row_stride};
     auto g = static_cast<const uint16_t*>(norm_g);
-    if (rows_form(a)) return launch_rows<false>(a, g, norm_eps, st);
+    if (!invariant && rows_form(a)) return launch_rows<false>(a, g, norm_eps, st);
     // chunks per lane NC = ceil(nch / 64), rounded up to an instantiated size; at most 16 loads per lane
     // (rows per wave measured on MI355X: 2 at K = 896; at K = 2048 1 up to N = 2048, 2 from N = 16 per CU on,
     // where each wave's activation row (and norm weights) from L2 then serves two weight rows: one token,

@@ -52,11 +52,10 @@ import thinker_attn as TA
 __all__ = ["FastThinkerStep"]
 
 _SCORING = ("sigmoid", "softmax")
-# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda); the engine switches its KDA layers' mode
-# past 192 (engine.py:946-949, 964-967), here both forms compute the same and the line lies where the chunked one is the
-# faster: us per layer's core at 16 / 32 / 64 / 150 / 192 rows 11.3 / 12.2 / 14.3 / 20.1 / 21.9 chunked, 10.8 / 13.9 /
-# 19.7 / 35.4 / 40.9 recurrent.
-KDA_CHUNK_ABOVE = 24
+# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda), as the engine switches its KDA layers'
+# mode (engine.py:946-949, 964-967). us per layer's core at 32 / 64 / 150 / 192 / 512 rows: 12.2 / 14.3 / 20.1 / 21.9 /
+# 43.7 chunked, 13.9 / 19.7 / 35.4 / 40.9 / 92.4 recurrent; shorter prompts keep the recurrent form's bits.
+KDA_CHUNK_ABOVE = 192
 
 
 def _norm(mod, what):
@@ -252,7 +251,7 @@ class FastThinkerStep:
         in_place: the residual is a buffer nobody reads afterwards, so the GEMM accumulates into it (beta = 1 on C = D,
         the same single rounding) instead of first copying it into a new output."""
         if x.shape[0] <= fastlinear.MAX_M:
-            return fastlinear.small_linear(x, w, b=b, residual=residual, norm=norm)
+            return fastlinear.small_linear(x, w, b=b, residual=residual, norm=norm, row_invariant=True)
         if norm is not None:
             x = fused_ops.rms_norm(x, norm[0], norm[1])
         if residual is not None and b is None:
@@ -264,8 +263,8 @@ class FastThinkerStep:
         """The attention half of layer li over a prompt's T rows h [T, H] at positions pos_buf .. pos_buf + T - 1:
         h + o(mixer(input_layernorm(h))). KDA: the projection, the q / k / v short convolutions (their caches end
         on the prompt's last real inputs), the f / g LoRA up-projections, the recurrence from the layer's state
-        (fused_recurrent_kda up to KDA_CHUNK_ABOVE rows, chunk_kda beyond; padding rows past n_valid leave the state
-        unchanged), rms_norm_gated; MLA: the
+        (fused_recurrent_kda up to KDA_CHUNK_ABOVE rows, chunk_kda beyond: the engine's mode switch,
+        engine.py:946-949; padding rows past n_valid leave the state unchanged), rms_norm_gated; MLA: the
         q | k | v projection and mla_prefill_attn (padding rows are stored past the real ones, where the next
         decode steps overwrite them before any query reads them). own: h is the step's and dead after this call, so
         the o projection past fastlinear.MAX_M rows adds into it in place."""
