@@ -299,6 +299,18 @@ __device__ __forceinline__ uint4 buf16(rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
 }
 
+// For memory that a launch reads once, the weights of a decode step above all: the nt bit, with which the lines are not
+// kept in the caches (a step streams more weights than these hold, so that keeping them only pushes out what is read
+// again). Cold decode blocks, us per layer with | without: bf16 one token 28.2 | 29.7, int8 21.2 | 23.4, bf16 8 tokens
+// 96.9 | 104.4; a Talker token 545 | 601, a 4-layer int8 thinker token 265 | 287.
+__device__ __forceinline__ uint4 buf16_once(rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 2));
+}
+__device__ __forceinline__ uint4 ld16_once(const uint16_t* p) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+}
+
 // With a wave-uniform part of the offset, which costs no vector instruction.
 __device__ __forceinline__ float4 buf16f(rsrc_t r, uint32_t off, uint32_t uniform) {
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), static_cast<int>(uniform), 0));
@@ -341,7 +353,12 @@ __device__ __forceinline__ void load_lds16(const void* src, char* lds_wave_base)
   __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)lds_wave_base, 16, 0, 0);
 }
 
-// The same through a buffer resource: a lane whose offset lies past the resource's end writes zeros to its LDS place.
+// The same for memory that this launch reads once: not kept in the caches (the nt bit).
+__device__ __forceinline__ void load_lds16_once(const void* src, char* lds_wave_base) {
+  __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)lds_wave_base, 16, 0, 2);
+}
+
+// load_lds16 through a buffer resource: a lane whose offset lies past the resource's end writes zeros to its LDS place.
 __device__ __forceinline__ void buf_lds16(rsrc_t r, uint32_t off, char* lds_wave_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds_wave_base, 16, static_cast<int>(off), 0, 0, 0);
 }

@@ -159,8 +159,8 @@ __device__ __forceinline__ void gate_up_one(const DecodeArgs& a, int e, int p, c
       for (int j = 0; j < NC; ++j) {
         const int64_t c = c0 + s + static_cast<int64_t>(LPR) * j;
         const bool ok = rok && c < nch;
-        wg[j] = buf16(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
-        wu[j] = buf16(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
+        wg[j] = buf16_once(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
+        wu[j] = buf16_once(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
       }
       Act<Q> xa[NC];
 #pragma unroll
@@ -227,8 +227,8 @@ __device__ __forceinline__ void gate_up_many_rows(const DecodeArgs& a, int e, in
     for (int j = 0; j < NC; ++j) {
       const int64_t c = s + static_cast<int64_t>(LPR) * j;
       const bool ok = rok && c < nch;
-      wg[j] = buf16(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
-      wu[j] = buf16(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
+      wg[j] = buf16_once(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
+      wu[j] = buf16_once(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
     }
   };
   // after group_sums a lane holds the gate total of the group's token vi < G (its up total, value G + vi, is at
@@ -315,8 +315,8 @@ __device__ __forceinline__ void gate_up_many(const DecodeArgs& a, int e, int cnt
     for (int j = 0; j < NC; ++j) {
       const int64_t c = s + static_cast<int64_t>(LPR) * j;
       const bool ok = rok && c < nch;
-      wg[j] = buf16(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
-      wu[j] = buf16(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
+      wg[j] = buf16_once(wr, ok ? goff + static_cast<uint32_t>(c) * 16u : kPast);
+      wu[j] = buf16_once(wr, ok ? uoff + static_cast<uint32_t>(c) * 16u : kPast);
     }
   }
   // stage the rows of this group's tokens and their zero padding (whole workgroup; the group is uniform across it),
@@ -531,7 +531,8 @@ __global__ __launch_bounds__(kDownWaves * 64) void decode_down_kernel(DecodeArgs
 #pragma unroll
           for (int j = 0; j < NC; ++j) {
             const int64_t c = s + static_cast<int64_t>(LPR) * j;
-            w[r][j] = buf16(wr, c < nch ? wrow + static_cast<uint32_t>(c) * 16u : kPast);
+            const uint32_t off = c < nch ? wrow + static_cast<uint32_t>(c) * 16u : kPast;
+            w[r][j] = ONE || !RELOAD ? buf16_once(wr, off) : buf16(wr, off);  // read again only by a batch's reloads
           }
         }
 #pragma unroll

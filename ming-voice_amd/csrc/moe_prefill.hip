@@ -104,9 +104,10 @@ struct PrefillArgs {
   int64_t ys;
 };
 
-// Tile of this workgroup: expert e, block blk (rows blk*BM ..), column tile nt. False: no tile.
+// Tile of this workgroup: expert e, block blk (rows blk*BM ..), column tile nt; once: the expert has this block only, so
+// no other tile reads its weight rows. False: no tile.
 template <int BM>
-__device__ __forceinline__ bool map_tile(const PrefillArgs& a, int NT, int& e, int& blk, int& nt) {
+__device__ __forceinline__ bool map_tile(const PrefillArgs& a, int NT, int& e, int& blk, int& nt, bool& once) {
   const int used_blocks = a.offsets[a.E1] / BM;
   const int G = used_blocks * NT;
   const int per = (G + kXcds - 1) / kXcds;
@@ -120,6 +121,7 @@ __device__ __forceinline__ bool map_tile(const PrefillArgs& a, int NT, int& e, i
   const int local = L - b0 * NT;
   nt = local / nblk;
   blk = b0 + local % nblk;
+  once = nblk == 1;
   return true;
 }
 
@@ -207,11 +209,12 @@ struct LoadMap {
 
 // Issues the direct loads of slab kt into LDS stage `st` (arow/brow: this thread's source row starts,
 // null for masked rows; k counted in elements; slab kt of an activation row starts kt * aslab elements in, of a
-// weight row kt * bslab).
-template <class G>
+// weight row kt * bslab). ONCE && once: no other tile reads these weights, and keeping them in the caches would only push
+// out what others share (few_pairs).
+template <class G, bool ONCE>
 __device__ __forceinline__ void issue_slab(char* lds, int st, int kt, int64_t K, const LoadMap<G>& m,
                                            const uint16_t* const* arow, const char* const* brow, int64_t aslab,
-                                           int64_t bslab) {
+                                           int64_t bslab, bool once) {
   constexpr int ES = G::Q ? 1 : 2;
   char* sa = lds + st * G::STAGE;
   char* sb = sa + G::A_BYTES;
@@ -227,7 +230,8 @@ __device__ __forceinline__ void issue_slab(char* lds, int st, int kt, int64_t K,
   for (int j = 0; j < G::B_INSTR; ++j) {
     const int64_t k = k0 + m.cb[j] * (16 / ES), kb = kt * bslab + m.cb[j] * (16 / ES);
     const void* src = (brow[j] && k < K) ? static_cast<const void*>(brow[j] + kb * ES) : static_cast<const void*>(g_zero_chunk);
-    load_lds16(src, sb + (w * G::B_INSTR + j) * 1024);
+    if (ONCE && once) load_lds16_once(src, sb + (w * G::B_INSTR + j) * 1024);
+    else load_lds16(src, sb + (w * G::B_INSTR + j) * 1024);
   }
 }
 
@@ -250,9 +254,10 @@ __device__ __forceinline__ int valid_rows(const int* spair, int P) {
 // where activation / weight row r's first slab starts and aslab / bslab the elements between its slabs. Row fragments at or
 // past fm_live (wave-uniform) hold only padding rows: their LDS reads and MFMAs are skipped and their
 // accumulators stay zero (the epilogues store no padding row).
-template <class G, class XRowFn, class WRowFn, class BColFn>
+template <class G, bool ONCE, class XRowFn, class WRowFn, class BColFn>
 __device__ __forceinline__ void tile_gemm(floatx4 (&acc)[G::FM][G::FN], int64_t K, XRowFn xrow, int64_t aslab,
-                                          WRowFn wrow, int64_t bslab, char* lds, int r0, BColFn bcol, int fm_live) {
+                                          WRowFn wrow, int64_t bslab, char* lds, int r0, BColFn bcol, int fm_live,
+                                          bool once) {
   constexpr int NS = G::NS, LOADS = G::LOADS, FM = G::FM, FN = G::FN;
   const int lane = lane_id();
   const int lr = lane & 15, lq = lane >> 4;
@@ -270,7 +275,7 @@ __device__ __forceinline__ void tile_gemm(floatx4 (&acc)[G::FM][G::FN], int64_t 
   const int nk = static_cast<int>((K + G::BK - 1) / G::BK);
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s)
-    if (s < nk) issue_slab<G>(lds, s, s, K, m, arow, brow, aslab, bslab);
+    if (s < nk) issue_slab<G, ONCE>(lds, s, s, K, m, arow, brow, aslab, bslab, once);
   for (int kt = 0; kt < nk; ++kt) {
     // slabs issued after kt so far: min(nk - 1 - kt, NS - 2); wait for kt's own loads
     const int pending = min(nk - 1 - kt, NS - 2);
@@ -285,7 +290,7 @@ __device__ __forceinline__ void tile_gemm(floatx4 (&acc)[G::FM][G::FN], int64_t 
     // slab kt visible to all waves; every wave is done with slab kt-1. A plain barrier: the loads of
     // slab kt were waited for above, and a memory fence would also wait for the later slabs' loads.
     __builtin_amdgcn_s_barrier();
-    if (kt + NS - 1 < nk) issue_slab<G>(lds, (kt + NS - 1) % NS, kt + NS - 1, K, m, arow, brow, aslab, bslab);
+    if (kt + NS - 1 < nk) issue_slab<G, ONCE>(lds, (kt + NS - 1) % NS, kt + NS - 1, K, m, arow, brow, aslab, bslab, once);
     const char* sa = lds + (kt % NS) * G::STAGE;
     const char* sb = sa + G::A_BYTES;
     if constexpr (G::Q) {
@@ -385,7 +390,7 @@ __device__ __forceinline__ void store_slab_rows(const uint16_t* ot, int os, cons
 // ------------------------------------------------------------------------------------------- gate / up
 
 // SL: the weights are the prefill copy of w_gu (kSlabRows-row pieces), else the row layout.
-template <bool Q, int BN, int NW, int BM, bool SL = false>
+template <bool Q, int BN, int NW, int BM, bool SL, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void prefill_gate_up_kernel(PrefillArgs a) {
   using G = Geo<Q, BN, NW, BM, !SL>;
   constexpr int HALF = G::BN / 2;  // gate columns per tile (and as many up columns)
@@ -393,7 +398,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_gate_up_kernel(PrefillArgs a)
   __shared__ int spair[BM];
   const int NT = static_cast<int>((a.I + HALF - 1) / HALF);
   int e, blk, nt;
-  if (!map_tile<BM>(a, NT, e, blk, nt)) return;
+  bool once;
+  if (!map_tile<BM>(a, NT, e, blk, nt, once)) return;
   constexpr int ES = Q ? 1 : 2;
   const int64_t I = a.I, n0 = static_cast<int64_t>(nt) * HALF;
   if (threadIdx.x < BM) spair[threadIdx.x] = a.sorted_ids[static_cast<int64_t>(blk) * BM + threadIdx.x];
@@ -419,8 +425,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_gate_up_kernel(PrefillArgs a)
   const int g0 = wn * FG * 16;       // first gate column of the wave, relative to n0
   floatx4 acc[G::FM][G::FN];
   const int fm_live = min(max((valid_rows<BM>(spair, a.P) - r0 + 15) / 16, 0), G::FM);
-  tile_gemm<G>(acc, a.H, xrow, G::BK, wrow, SL ? R * G::BK : G::BK, reinterpret_cast<char*>(lds_raw), r0,
-               [&](int j) { return (j < FG ? 0 : HALF) + g0 + 16 * (j % FG); }, fm_live);
+  tile_gemm<G, ONCE>(acc, a.H, xrow, G::BK, wrow, SL ? R * G::BK : G::BK, reinterpret_cast<char*>(lds_raw), r0,
+               [&](int j) { return (j < FG ? 0 : HALF) + g0 + 16 * (j % FG); }, fm_live, once);
   // the output tile [BM][HALF] goes through LDS (free once every wave is past the last slab), then out in rows
   constexpr int OS = HALF + 8;  // row stride (elements): rows 4 apart start 64 bytes apart on the banks
   static_assert(static_cast<size_t>(BM) * OS * 2 <= G::LDS, "gate/up output tile must fit in the k-slab LDS");
@@ -466,14 +472,15 @@ __global__ __launch_bounds__(NW * 64) void prefill_gate_up_kernel(PrefillArgs a)
 // ----------------------------------------------------------------------------------------------- down
 
 // SL: the weights are the prefill copy of w_d (kSlabRows-row pieces), else the row layout.
-template <bool Q, int BN, int NW, int BM, bool SL = false>
+template <bool Q, int BN, int NW, int BM, bool SL, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void prefill_down_kernel(PrefillArgs a) {
   using G = Geo<Q, BN, NW, BM>;
   extern __shared__ uint4 lds_raw[];
   __shared__ int spair[BM];
   const int NT = static_cast<int>((a.H + G::BN - 1) / G::BN);
   int e, blk, nt;
-  if (!map_tile<BM>(a, NT, e, blk, nt)) return;
+  bool once;
+  if (!map_tile<BM>(a, NT, e, blk, nt, once)) return;
   constexpr int ES = Q ? 1 : 2;
   const int64_t H = a.H, I = a.I, h0 = static_cast<int64_t>(nt) * G::BN;
   if (threadIdx.x < BM) spair[threadIdx.x] = a.sorted_ids[static_cast<int64_t>(blk) * BM + threadIdx.x];
@@ -498,8 +505,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_down_kernel(PrefillArgs a) {
   const int c0 = wn * G::FN * 16;
   floatx4 acc[G::FM][G::FN];
   const int fm_live = min(max((valid_rows<BM>(spair, a.P) - r0 + 15) / 16, 0), G::FM);
-  tile_gemm<G>(acc, I, xrow, MM_PREFILL_A_SLABS ? BM * 64 : G::BK, wrow, SL ? R * G::BK : G::BK,
-               reinterpret_cast<char*>(lds_raw), r0, [&](int j) { return c0 + 16 * j; }, fm_live);
+  tile_gemm<G, ONCE>(acc, I, xrow, MM_PREFILL_A_SLABS ? BM * 64 : G::BK, wrow, SL ? R * G::BK : G::BK,
+               reinterpret_cast<char*>(lds_raw), r0, [&](int j) { return c0 + 16 * j; }, fm_live, once);
   // the output tile [BM][BN] goes through LDS, then out in rows (as in gate/up)
   constexpr int OS = G::BN + 8;
   static_assert(static_cast<size_t>(BM) * OS * 2 <= G::LDS, "down output tile must fit in the k-slab LDS");
@@ -613,31 +620,38 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
 
 constexpr int kCombineMaxK = 16;
 
-template <bool Q, int BN, int NW, int BM, bool SL>
+template <bool Q, int BN, int NW, int BM, bool SL, bool ONCE>
 int launch_gate_up(const PrefillArgs& a, int64_t nb, hipStream_t st) {
   using G = Geo<Q, BN, NW, BM, !SL>;
   const int64_t nt = (a.I + G::BN / 2 - 1) / (G::BN / 2);
   const int64_t g = (nb * nt + kXcds - 1) / kXcds * kXcds;
-  int rc = mm::allow_lds(prefill_gate_up_kernel<Q, BN, NW, BM, SL>, G::LDS, "prefill_gate_up");
+  int rc = mm::allow_lds(prefill_gate_up_kernel<Q, BN, NW, BM, SL, ONCE>, G::LDS, "prefill_gate_up");
   if (rc) return rc;
-  hipLaunchKernelGGL((prefill_gate_up_kernel<Q, BN, NW, BM, SL>), dim3(static_cast<unsigned>(g)), dim3(NW * 64), G::LDS,
+  hipLaunchKernelGGL((prefill_gate_up_kernel<Q, BN, NW, BM, SL, ONCE>), dim3(static_cast<unsigned>(g)), dim3(NW * 64), G::LDS,
                      st, a);
   return mm::check_launch("moe_prefill gate_up");
 }
 
-template <bool Q, int BN, int NW, int BM, bool SL>
+template <bool Q, int BN, int NW, int BM, bool SL, bool ONCE>
 int launch_down(const PrefillArgs& a, int64_t nb, hipStream_t st) {
   using G = Geo<Q, BN, NW, BM>;
   const int64_t nt = (a.H + G::BN - 1) / G::BN;
   const int64_t g = (nb * nt + kXcds - 1) / kXcds * kXcds;
-  int rc = mm::allow_lds(prefill_down_kernel<Q, BN, NW, BM, SL>, G::LDS, "prefill_down");
+  int rc = mm::allow_lds(prefill_down_kernel<Q, BN, NW, BM, SL, ONCE>, G::LDS, "prefill_down");
   if (rc) return rc;
-  hipLaunchKernelGGL((prefill_down_kernel<Q, BN, NW, BM, SL>), dim3(static_cast<unsigned>(g)), dim3(NW * 64), G::LDS, st,
+  hipLaunchKernelGGL((prefill_down_kernel<Q, BN, NW, BM, SL, ONCE>), dim3(static_cast<unsigned>(g)), dim3(NW * 64), G::LDS, st,
                      a);
   return mm::check_launch("moe_prefill down");
 }
 
-template <bool Q, int BM>
+// Experts averaging few pairs mostly have one block, so that a tile's weight rows are no other's: the variants that load
+// those past the caches (ONCE). Above, most weights are shared, and the test alone costs the kernels 2 %. Block us with |
+// without: 64 experts, 4 / 16 / 28 pairs each 180 | 194, 215 | 229, 232 | 247, int8 110 | 114, 136 | 145; 38 / 43 / 48
+// 238 | 248, 240 | 246, 243 | 246; 55 247 | 246, int8 110 252 | 241; 128 experts, 21 / 35 / 49 152 | 162, 154 | 165,
+// 165 | 172. (For every tile's weights, shared or not, 512 tokens took 265 us instead of 248.)
+bool few_pairs(const PrefillArgs& a) { return a.P < static_cast<int64_t>(48) * a.E1; }
+
+template <bool Q, int BM, bool ONCE>
 int launch_gemms(const PrefillArgs& a, int64_t nb, int phases, hipStream_t st) {
   constexpr int GU_BN = Q ? MM_PREFILL_GU_BN_INT8 : MM_PREFILL_GU_BN_BF16;
   constexpr int DOWN_BN = Q ? MM_PREFILL_DOWN_BN_INT8 : MM_PREFILL_DOWN_BN_BF16;
@@ -645,11 +659,13 @@ int launch_gemms(const PrefillArgs& a, int64_t nb, int phases, hipStream_t st) {
   constexpr int DOWN_NW = Q ? MM_PREFILL_DOWN_WAVES_INT8 : MM_PREFILL_DOWN_WAVES_BF16;
   int rc;
   if (phases & MM_PHASE_GATE_UP) {
-    rc = a.gu_slabs ? launch_gate_up<Q, GU_BN, GU_NW, BM, true>(a, nb, st) : launch_gate_up<Q, GU_BN, GU_NW, BM, false>(a, nb, st);
+    rc = a.gu_slabs ? launch_gate_up<Q, GU_BN, GU_NW, BM, true, ONCE>(a, nb, st)
+                    : launch_gate_up<Q, GU_BN, GU_NW, BM, false, ONCE>(a, nb, st);
     if (rc) return rc;
   }
   if (phases & MM_PHASE_DOWN) {
-    rc = a.d_slabs ? launch_down<Q, DOWN_BN, DOWN_NW, BM, true>(a, nb, st) : launch_down<Q, DOWN_BN, DOWN_NW, BM, false>(a, nb, st);
+    rc = a.d_slabs ? launch_down<Q, DOWN_BN, DOWN_NW, BM, true, ONCE>(a, nb, st)
+                   : launch_down<Q, DOWN_BN, DOWN_NW, BM, false, ONCE>(a, nb, st);
     if (rc) return rc;
   }
   return MM_OK;
@@ -809,9 +825,11 @@ extern "C" int mm_moe_prefill(const void* x, int64_t n_tokens, int64_t x_row_str
   hipStream_t st = MM_STREAM(stream);
   if (phases == MM_PHASE_ALL) phases = MM_PHASE_GATE_UP | MM_PHASE_DOWN | MM_PHASE_COMBINE;
   if (nb > 0) {
-    if (ex->w_dtype == MM_INT8) rc = launch_gemms<true, kBMSmall>(a, nb, phases, st);
-    else if (block_m == kBM) rc = launch_gemms<false, kBM>(a, nb, phases, st);
-    else rc = launch_gemms<false, kBMSmall>(a, nb, phases, st);
+    const bool few = few_pairs(a);
+    if (ex->w_dtype == MM_INT8)
+      rc = few ? launch_gemms<true, kBMSmall, true>(a, nb, phases, st) : launch_gemms<true, kBMSmall, false>(a, nb, phases, st);
+    else if (block_m == kBM) rc = launch_gemms<false, kBM, false>(a, nb, phases, st);
+    else rc = few ? launch_gemms<false, kBMSmall, true>(a, nb, phases, st) : launch_gemms<false, kBMSmall, false>(a, nb, phases, st);
     if (rc) return rc;
   }
   if (!(phases & MM_PHASE_COMBINE)) return MM_OK;

@@ -146,7 +146,10 @@ __global__ __launch_bounds__(256) void small_linear_1pass_kernel(LinArgs a, cons
   for (int i = 0; i < R; ++i) {
     const int64_t nl = wrow(i);
 #pragma unroll
-    for (int j = 0; j < NC; ++j) w[i][j] = *reinterpret_cast<const uint4*>(a.w + nl * a.ws + cc[j] * 8);
+    for (int j = 0; j < NC; ++j) {
+      const uint16_t* p = a.w + nl * a.ws + cc[j] * 8;
+      w[i][j] = MG == 1 ? ld16_once(p) : *reinterpret_cast<const uint4*>(p);  // a decode step's weights: see ld16_once
+    }
   }
   uint4 gv[NC];
   if constexpr (NORM) {
