@@ -792,7 +792,7 @@ def main():
                                       "the call)",
                    "down_weights": "prefill copy of the down stack (the same)",
                    "copy_bytes_per_layer": b_copy_bytes},
-        "roofline": {"bound": "hbm", "kernel": "prefill_gate_up_kernel<false, 128, 8, 64, true>", "achieved": achieved,
+        "roofline": {"bound": "hbm", "kernel": "prefill_gate_up_kernel<false, 128, 8, 64, true, false>", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic},
         "cpu_baseline": cpu,
         "box": box_info(),
