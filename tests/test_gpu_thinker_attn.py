@@ -313,6 +313,20 @@ def test_mla_decode_attn_matches_oracle(nh, dq, dv, L):
         assert torch.equal(kc[0].cpu(), rk) and torch.equal(vc[0].cpu(), rv)
 
 
+@pytest.mark.parametrize("nh,dq,dv", [(2, 192, 128), (1, 32, 40), (1, 64, 256)])
+@pytest.mark.parametrize("pos", [1023, 1024, 1151, 1152, 3071, 3072, 3199])
+def test_mla_decode_attn_at_the_edges_of_the_merge_batches(nh, dq, dv, pos):
+    """The merge takes 8 chunks of 32 positions per wave at first (up to 1023), then 16 per wave (up to 3071, ...);
+    a workspace of NaN shows that no chunk past the position enters."""
+    kc = W.normal((1, nh, 3200, dq), 1.0, 422, DEV)
+    vc = W.normal((1, nh, 3200, dv), 1.0, 423, DEV)
+    q, kn, vn = W.normal((nh, dq), 1.0, 424, DEV), W.normal((nh, dq), 1.0, 425, DEV), W.normal((nh, dv), 1.0, 426, DEV)
+    ro, _, _ = A.mla_decode_attn(q.cpu(), kn.cpu(), vn.cpu(), kc[0].cpu(), vc[0].cpu(), pos)
+    ws = TA.mla_attn_workspace(nh, dv, 3200, DEV)
+    ws.view(torch.uint8).fill_(0xff)
+    close(TA.mla_decode_attn(q, kn, vn, kc, vc, torch.tensor([pos], device=DEV), workspace=ws), ro)
+
+
 def test_mla_rows_past_the_position_are_never_read():
     """Cache rows past pos filled with NaN (an uninitialised cache) leave the output finite and equal to the
     oracle's; the last position of a partial chunk and of the cache included."""
