@@ -1709,7 +1709,7 @@ __device__ __forceinline__ int mla_v_chunk(int row, int c) {
 // softmax(scale q_t . K[0..pos+t]^T) . V[0..pos+t] (engine.py:679-682's mask), rows below pos from the cache, the
 // prompt's own from k_new / v_new, which the workgroup of a token's queries also copies to its cache row
 // (engine.py:537-541; no workgroup reads those cache rows, so the copy needs no launch of its own). a.stored: the rows
-// are in the cache already (mla_prefill_store_kernel) and are read there.
+// are in the cache already (mla_prefill_store_kernel) and are read there, k_new and v_new by nobody.
 // Grid (nh, query blocks, the last and longest first) x NW waves: with 8 or more heads the workgroups of a head share an
 // XCD, whose L2 then serves its keys and values. A workgroup holds 16 QF queries of one head, and its waves take the
 // 32-key tiles round robin (wave w: tiles w, w + NW, ...; first the cached keys' tiles, then the prompt's), each keeping
@@ -2357,9 +2357,16 @@ extern "C" int mm_mla_prefill_attn(const void* q, int64_t q_ts, const void* k_ne
   a.out = static_cast<uint16_t*>(out);
   a.out_ts = out_ts;
   hipStream_t st = MM_STREAM(stream);
-  // the attention kernel addresses a tile's 32 rows by 32-bit offsets; token strides past that (2^25 elements) store the
-  // rows first and read them from the cache
-  a.stored = k_ts >= (1 << 25) || v_ts >= (1 << 25);
+  // Two calls store the rows first and read them from the cache: token strides past 2^25 elements, since the attention
+  // kernel addresses a tile's 32 rows by 32-bit offsets, and an out that meets k_new or v_new (the values' buffer used
+  // again for the result: both are nh dv wide), since a workgroup reads the rows of all earlier tokens while others
+  // already store their outputs. Spans are compared, so column slices of one buffer count as meeting.
+  auto meets_out = [&](const void* p, int64_t ts, int d) {
+    const auto b = reinterpret_cast<uintptr_t>(p), o = reinterpret_cast<uintptr_t>(out);
+    const int64_t row = static_cast<int64_t>(nh) * d, orow = static_cast<int64_t>(nh) * dv;
+    return b < o + static_cast<uintptr_t>((T - 1) * out_ts + orow) * 2 && o < b + static_cast<uintptr_t>((T - 1) * ts + row) * 2;
+  };
+  a.stored = k_ts >= (1 << 25) || v_ts >= (1 << 25) || meets_out(k_new, k_ts, dqk) || meets_out(v_new, v_ts, dv);
   if (a.stored) {
     hipLaunchKernelGGL(mla_prefill_store_kernel, dim3(static_cast<unsigned>(T), static_cast<unsigned>(nh)), dim3(kWave),
                        0, st, a);

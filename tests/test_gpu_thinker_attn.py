@@ -484,6 +484,26 @@ def test_mla_prefill_values_past_a_query_block_and_far_token_strides():
     assert torch.equal(ke, kf) and torch.equal(ve, vf)
 
 
+@pytest.mark.parametrize("T,pos", [(1, 5), (33, 31), (300, 40), (544, 10)])
+@pytest.mark.parametrize("over", ["v", "v shifted", "k"])
+def test_mla_prefill_out_over_the_new_rows(T, pos, over):
+    """out in the buffer of v_new or k_new, or reaching into it, for every shape of the workgroups: the result and the
+    caches of a separate out, bit for bit."""
+    nh, dq, dv = 16, 192, 128
+    print(f"[mla prefill out over {over}] T={T} pos={pos}", flush=True)
+    kc = W.normal((1, nh, T + pos, dq), 1.0, 550, DEV)
+    vc = W.normal((1, nh, T + pos, dv), 1.0, 551, DEV)
+    q, kn, vn = (x.reshape(T, -1) for x in _prompt(nh, dq, dv, T, 552))
+    buf = torch.empty(T * nh * dv + 64, device=DEV, dtype=BF)  # v_new, with room for an out 64 elements further on
+    vn = buf[:T * nh * dv].view(T, nh * dv).copy_(vn)
+    k2, v2, p = kc.clone(), vc.clone(), torch.tensor([pos], device=DEV)
+    want = TA.mla_prefill_attn(q, kn, vn, k2, v2, p)
+    out = {"v": vn, "v shifted": buf[64:].view(T, nh * dv), "k": kn.reshape(-1)[:T * nh * dv].view(T, nh * dv)}[over]
+    got = TA.mla_prefill_attn(q, kn, vn, kc, vc, p, out=out)
+    assert got.data_ptr() == out.data_ptr() and torch.equal(got, want)
+    assert torch.equal(kc, k2) and torch.equal(vc, v2)
+
+
 def test_mla_prefill_one_token_equals_decode_and_graph_replays_follow_the_position():
     nh, dq, dv, L = 16, 192, 128, 512
     kc = W.normal((1, nh, L, dq), 1.0, 520, DEV)
