@@ -534,8 +534,8 @@ __global__ __launch_bounds__(2 * K, 3) void kda_chunk_prep_kernel(KdaArgs a, flo
   if (a.use_gate && isnan(a.lower_bound)) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float x = d[e] + dt[e], y = log1pf(__expf(fminf(x, 20.f)));
-      d[e] = -nA * (x > 20.f ? x : y);
+      const float x = d[e] + dt[e], y = log1pf(__expf(x));
+      d[e] = -nA * (x > 20.f ? x : y);  // an x that is NaN gives y, NaN
     }
   } else if (a.use_gate) {
 #pragma unroll

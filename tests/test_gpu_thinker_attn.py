@@ -114,6 +114,27 @@ def test_kda_chunk_nan_padding_and_far_token_strides():
     assert torch.equal(a, b) and torch.equal(fa, fb)
 
 
+@pytest.mark.parametrize("where", ["g", "dt_bias"])
+@pytest.mark.parametrize("lb", [None, -5.0])
+def test_kda_chunk_nan_gate_reaches_the_state(where, lb):
+    """A NaN in one channel's gate of a real token, or in its dt_bias, makes the head's state and its outputs from that
+    token on NaN in chunk_kda as in fused_recurrent_kda; the other heads keep their bits."""
+    T, t, H, K, V = 40, 21, 3, 128, 32
+    print(f"[kda nan gate] {where} lb={lb}", flush=True)
+    q, k, v, g, beta, A_log, dt, S0 = _kda_inputs(T, H, K, V, 940)
+    kw = dict(A_log=A_log, initial_state=S0, use_qk_l2norm_in_kernel=True, use_gate_in_kernel=True, lower_bound=lb,
+              output_final_state=True)
+    ok = {fn: fn(q, k, v, g, beta, dt_bias=dt, **kw) for fn in (TA.chunk_kda, TA.fused_recurrent_kda)}
+    if where == "g":
+        g[0, t, 1, 5] = float("nan")
+    else:
+        dt[K + 5], t = float("nan"), 0
+    for fn, (o0, s0) in ok.items():
+        o, s = fn(q, k, v, g, beta, dt_bias=dt, **kw)
+        assert torch.isnan(s[0, 1]).all() and torch.isnan(o[0, t:, 1].float()).all(), fn.__name__
+        assert torch.equal(s[0, [0, 2]], s0[0, [0, 2]]) and torch.equal(o[0, :, [0, 2]], o0[0, :, [0, 2]]), fn.__name__
+
+
 def test_kda_chunk_full_prompt_and_strong_decay():
     """The hybrid thinker's shape, 512 tokens over 16 heads of 128 x 128, against the float64 recurrence; then decays
     of e^-30 .. e^-80 per token, whose products over a chunk underflow: the chunk form takes them as products, never
