@@ -21,7 +21,7 @@
 extern "C" {
 #endif
 
-#define MM_ABI_VERSION 16
+#define MM_ABI_VERSION 17
 
 /* status codes */
 #define MM_OK 0

@@ -1,6 +1,7 @@
 """CPU checks of the C ABI: the library loads and exports every entry point of include/mingmoe.h, the
 ctypes struct matches the C layout, and argument validation fails with a message before any GPU work."""
 import ctypes
+import hashlib
 import os
 import re
 import subprocess
@@ -28,6 +29,19 @@ def test_library_exports_every_declared_symbol():
     for name in _declared():
         assert hasattr(lib, name), name
     assert lib.mm_version() == mm.ABI_VERSION
+
+
+# digests of the header's interface (macros, types, prototypes; no comments) by version: a change of the interface comes
+# with a new version and its digest, so that a library built before it is refused when it is loaded
+INTERFACES = {16: "b5dd488052f53fa4", 17: "b5df4bc6e101d7db"}
+
+
+def test_the_version_moves_with_the_interface():
+    text = re.sub(r"/\*.*?\*/", " ", open(HEADER).read(), flags=re.S)
+    version = int(re.search(r"#define MM_ABI_VERSION (\d+)", text).group(1))
+    code = " ".join(re.sub(r"#define MM_ABI_VERSION \d+", "", text).split())
+    assert hashlib.sha256(code.encode()).hexdigest()[:16] == INTERFACES[version]
+    assert version == mm.ABI_VERSION == max(INTERFACES)
 
 
 def test_experts_struct_layout_matches_c(tmp_path):
