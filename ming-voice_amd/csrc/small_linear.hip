@@ -117,10 +117,14 @@ constexpr int row_group(int NC) { return NC <= 2 ? 8 : NC <= 4 ? 4 : NC <= 8 ? 2
 // silu_mul (fast_talker.py:258-260), bit for bit, without the [M, 2N] intermediate.
 // SPLIT: each workgroup takes the one token group blockIdx.y of a grid with a y row per group; otherwise it
 // takes every group in turn.
-template <int NC, int R, bool NORM, bool GLU, int MG, bool SPLIT = false>
+// ONE: a single token row, a decode step's: its weights are read past the caches (ld16_once). Not for several rows, also
+// where they go one at a time (K > 4096): SPLIT's workgroups share a weight row through the caches. us with that | without,
+// 2 rows: 6144 -> 2048 10.6 | 8.8 from memory and 6.3 | 5.5 from the caches, 4 rows: 4864 -> 896 7.2 | 6.4 from memory.
+template <int NC, int R, bool NORM, bool GLU, int MG, bool SPLIT, bool ONE>
 __global__ __launch_bounds__(256) void small_linear_1pass_kernel(LinArgs a, const uint16_t* __restrict__ norm_g,
                                                                  float norm_eps) {
   static_assert(!GLU || R == 2, "GLU pairs a gate row with an up row");
+  static_assert(!ONE || (MG == 1 && !SPLIT), "one token row");
   static_assert(MG * R <= kWave, "one epilogue lane per (token row, output row)");
   constexpr bool kShareNorm = NORM && MG > 1;
   constexpr int OUTS = GLU ? 1 : R;  // output rows per wave
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(256) void small_linear_1pass_kernel(LinArgs a, cons
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const uint16_t* p = a.w + nl * a.ws + cc[j] * 8;
-      w[i][j] = MG == 1 ? ld16_once(p) : *reinterpret_cast<const uint4*>(p);  // a decode step's weights: see ld16_once
+      w[i][j] = ONE ? ld16_once(p) : *reinterpret_cast<const uint4*>(p);
     }
   }
   uint4 gv[NC];
@@ -485,7 +489,7 @@ __global__ __launch_bounds__(256) void small_linear_kernel(LinArgs a) {
   }
 }
 
-template <int NC, int R, bool GLU, int MG>
+template <int NC, int R, bool GLU, int MG, bool ONE>
 void launch_1pass_mg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
   // Several token groups run in parallel workgroups (grid y) when the whole grid fits on the GPU at once: the
   // workgroups of one row block then read its weights together (one HBM read), where one workgroup taking the
@@ -493,22 +497,23 @@ void launch_1pass_mg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t
   // since workgroups of the same rows that are not resident together would each stream the weights.
   const unsigned gx = static_cast<unsigned>(GLU ? (a.N + 3) / 4 : (a.N + 4 * R - 1) / (4 * R));
   const unsigned ng = static_cast<unsigned>((a.M + MG - 1) / MG);
-  const bool split = ng > 1 && static_cast<int64_t>(gx) * ng <= static_cast<int64_t>(4) * mm::cu_count();
-  if (split) {
-    const dim3 grid(gx, ng);
-    if (g) hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, true, GLU, MG, true>), grid, dim3(256), 0, st, a, g, eps);
-    else hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, false, GLU, MG, true>), grid, dim3(256), 0, st, a, g, eps);
-    return;
+  if constexpr (!ONE) {
+    if (ng > 1 && static_cast<int64_t>(gx) * ng <= static_cast<int64_t>(4) * mm::cu_count()) {
+      const dim3 grid(gx, ng);
+      if (g) hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, true, GLU, MG, true, false>), grid, dim3(256), 0, st, a, g, eps);
+      else hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, false, GLU, MG, true, false>), grid, dim3(256), 0, st, a, g, eps);
+      return;
+    }
   }
   const dim3 grid(gx);
-  if (g) hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, true, GLU, MG>), grid, dim3(256), 0, st, a, g, eps);
-  else hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, false, GLU, MG>), grid, dim3(256), 0, st, a, g, eps);
+  if (g) hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, true, GLU, MG, false, ONE>), grid, dim3(256), 0, st, a, g, eps);
+  else hipLaunchKernelGGL((small_linear_1pass_kernel<NC, R, false, GLU, MG, false, ONE>), grid, dim3(256), 0, st, a, g, eps);
 }
 
 template <int NC, int R, bool GLU = false>
 int launch_1pass(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  if (a.M == 1) launch_1pass_mg<NC, R, GLU, 1>(a, g, eps, st);
-  else launch_1pass_mg<NC, R, GLU, row_group(NC)>(a, g, eps, st);
+  if (a.M == 1) launch_1pass_mg<NC, R, GLU, 1, true>(a, g, eps, st);
+  else launch_1pass_mg<NC, R, GLU, row_group(NC), false>(a, g, eps, st);
   return mm::check_launch(GLU ? "small_linear_glu" : "small_linear");
 }
 
