@@ -21,7 +21,7 @@
 extern "C" {
 #endif
 
-#define MM_ABI_VERSION 17
+#define MM_ABI_VERSION 18
 
 /* status codes */
 #define MM_OK 0
@@ -55,7 +55,9 @@ extern "C" {
 /* ORed into small_linear's act: the norm prologue rounds once, bf16(x * rstd * g), as torch's F.rms_norm does on
  * the reference's path for more than 16 rows (fastlinear.py:151-160), instead of bf16(bf16(x * rstd) * g). */
 #define MM_NORM_ROUND_ONCE 0x100
-#define MM_ROW_INVARIANT 0x200
+/* ORed into small_linear's act: 2 to 16 rows of up to 4096 elements may take the matrix units, whose sums run in another
+ * order. Without it every row gets the bits it gets with M = 1, whatever rows come with it. */
+#define MM_ANY_SUM_ORDER 0x400
 
 /* Stacked expert weights, as the thinker lays them out (engine.py:150-188, 313-391):
  *   w_gu [n_slots, 2*inter, hidden]  rows 0..inter-1 = gate, inter..2*inter-1 = up
@@ -225,8 +227,8 @@ int mm_moe_block_prefill(const void* x, int64_t n_tokens, int64_t x_row_stride, 
  * x, w, b, residual, norm_g, y: bf16. norm_g (optional): RMSNorm prologue with norm_eps,
  * x -> bf16(bf16(x * rstd) * g), or bf16(x * rstd * g) with MM_NORM_ROUND_ONCE in act (the rounding of the
  * reference's torch path for M > 16, which callers run as 16-row pieces). b, residual, norm_g may be NULL.
- * act: MM_ACT_* (| MM_NORM_ROUND_ONCE | MM_ROW_INVARIANT: every row gets the bits it gets with M = 1, whatever rows
- * come with it; without it several rows may take the matrix units, whose sums run in another order).
+ * act: MM_ACT_* (| MM_NORM_ROUND_ONCE | MM_ANY_SUM_ORDER). Every row gets the bits it gets with M = 1 unless the latter
+ * is given.
  * xn_buf: bf16 scratch [M, K], used only when a norm prologue is given and K > 8192 (may be NULL otherwise);
  * shorter rows get the norm fused into the GEMV. x_row_stride 0 repeats one activation row M times. */
 int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_row_stride,
@@ -237,7 +239,8 @@ int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_row_stride,
 
 /* act = silu_mul(small_linear(norm?(x), W)) in one kernel: W [2*inter, K] holds the gate rows then the up
  * rows; y[:, p] = bf16(bf16(silu(g_p)) * u_p) with g_p, u_p the bf16-rounded projections of rows p and
- * inter + p, so the result equals small_linear followed by silu_mul bit for bit. No counterpart in the
+ * inter + p, so the result equals small_linear (without MM_ANY_SUM_ORDER) followed by silu_mul bit for bit, and every
+ * row gets the bits it gets with M = 1. No counterpart in the
  * reference: it fuses fast_talker.py:258-260 (gate|up small_linear, _silu_mul) for callers that own the
  * layer loop. x, w, norm_g, y: bf16; M <= 16; K <= 8192, a multiple of 8; norm_g may be NULL. */
 int mm_small_linear_glu(const void* x, int64_t M, int64_t K, int64_t x_row_stride, const void* w, int64_t inter,

@@ -1,7 +1,7 @@
 // Small-M linear, M <= 16 (fastlinear.py:123-174): y = act(norm?(x) . W^T + b) [+ residual].
-// HBM-bound GEMV, latency-bound at decode sizes (a few MB per call). Several rows of up to 4096 elements take the matrix
-// units (small_linear_rows_kernel, below) unless each is to get the bits it gets alone (MM_ROW_INVARIANT: the thinker's
-// short prompts); one row, and longer ones, the vector form. For rows of up to 1024 16-byte chunks
+// HBM-bound GEMV, latency-bound at decode sizes (a few MB per call). Every row gets the bits it gets alone, whatever rows
+// come with it; a caller that does without that (MM_ANY_SUM_ORDER: the Talker's tail) has several rows of up to 4096
+// elements on the matrix units (small_linear_rows_kernel, below). For rows of up to 1024 16-byte chunks
 // (K <= 8192) one pass covers the row: a wave shares each of its rows across its 64 lanes and issues all
 // weight loads of its rows at once, so it waits for memory once; the activation chunks come from the L1/L2
 // caches. The optional RMSNorm prologue is fused there: the lanes of a wave hold the whole activation row,
@@ -272,12 +272,11 @@ __global__ __launch_bounds__(256) void small_linear_1pass_kernel(LinArgs a, cons
 // us per launch (rows: K -> N, n with the norm fused), the vector form -> this one: 6: 1024 -> 3072 n 5.6 -> 4.2, 1024 ->
 // 1024 3.2 -> 2.5, 1024 -> 4096 n 6.3 -> 4.6, 4096 -> 1024 5.5 -> 4.6; 2: 1024 -> 3072 n 4.6 -> 3.4; 16: 2048 -> 6416 n
 // 26.2 -> 17.3, 2048 -> 2048 9.3 -> 5.4 (a launch alone is about 2).
-template <int NC, int TG, int RQ, bool NORM, bool GLU>
+template <int NC, int TG, int RQ, bool NORM>
 __global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const uint16_t* __restrict__ norm_g,
                                                                 float norm_eps) {
-  static_assert(!GLU || RQ == 2, "GLU: a quad of gate rows and its quad of up rows");
   constexpr int V = RQ * TG * 4;             // totals per lane group: (weight quad q, token group t, weight row) in order
-  constexpr int NR = GLU ? 4 : 4 * RQ;       // output columns of the workgroup
+  constexpr int NR = 4 * RQ;                 // output columns of the workgroup
   __shared__ float s_ss[4][TG * 4];
   __shared__ float s_part[4][V][4];
   const int lane = lane_id(), wave = threadIdx.x / kWave, b = lane >> 2, r = lane & 3;
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const
   }
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
-    const int64_t row = GLU ? n0 + q * a.N : n0 + 4 * q, left = GLU ? a.N - n0 : a.N - row;  // its rows: 4 at most
+    const int64_t row = n0 + 4 * q, left = a.N - row;  // its rows: 4 at most
     const rsrc_t wr = make_rsrc(a.w + (left > 0 ? row : 0) * a.ws, left > 0 ? ((min(left, static_cast<int64_t>(4)) - 1) * a.ws + a.K) * 2 : 0);
 #pragma unroll
     for (int j = 0; j < NC; ++j) wv[q][j] = buf16(wr, c16[j] == kPast ? kPast : static_cast<uint32_t>(r * a.ws) * 2u + c16[j]);
@@ -311,8 +310,8 @@ __global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const
   // this thread's output: token row em, column n0 + en
   const int em = threadIdx.x / NR, en = threadIdx.x % NR;
   const bool live = em < a.M && n0 + en < a.N;
-  const rsrc_t br = make_rsrc(a.b, !GLU && a.b ? a.N * 2 : 0);
-  const rsrc_t rr = make_rsrc(a.res, !GLU && a.res ? ((a.M - 1) * a.rs + a.N) * 2 : 0);
+  const rsrc_t br = make_rsrc(a.b, a.b ? a.N * 2 : 0);
+  const rsrc_t rr = make_rsrc(a.res, a.res ? ((a.M - 1) * a.rs + a.N) * 2 : 0);
   const float bias = bf16_to_f32(buf2(br, live ? static_cast<uint32_t>(n0 + en) * 2u : kPast));
   const float res = bf16_to_f32(buf2(rr, live ? static_cast<uint32_t>(em * a.rs + n0 + en) * 2u : kPast));
   if constexpr (NORM) {
@@ -386,47 +385,38 @@ __global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const
     return ((s_part[0][v][em % 4] + s_part[1][v][em % 4]) + s_part[2][v][em % 4]) + s_part[3][v][em % 4];
   };
   uint16_t* y = a.y + em * a.ys + n0 + en;
-  if constexpr (GLU) {
-    *y = f32_to_bf16(round_bf16(silu(round_bf16(total(0, en)))) * round_bf16(total(1, en)));
-  } else {
-    const float keep = total(en / 4, en % 4);
-    float v = apply_act(a.b ? keep + bias : keep, a.act);
-    if (a.res) v = round_bf16(v) + res;
-    *y = f32_to_bf16(v);
-  }
+  const float keep = total(en / 4, en % 4);
+  float v = apply_act(a.b ? keep + bias : keep, a.act);
+  if (a.res) v = round_bf16(v) + res;
+  *y = f32_to_bf16(v);
 }
 
-template <int NC, int TG, int RQ, bool GLU>
+template <int NC, int TG, int RQ>
 int launch_rows_rq(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  constexpr int NR = GLU ? 4 : 4 * RQ;
-  const dim3 grid(static_cast<unsigned>((a.N + NR - 1) / NR));
-  if (g) hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, true, GLU>), grid, dim3(256), 0, st, a, g, eps);
-  else hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, false, GLU>), grid, dim3(256), 0, st, a, g, eps);
-  return mm::check_launch(GLU ? "small_linear_glu" : "small_linear");
+  const dim3 grid(static_cast<unsigned>((a.N + 4 * RQ - 1) / (4 * RQ)));
+  if (g) hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, true>), grid, dim3(256), 0, st, a, g, eps);
+  else hipLaunchKernelGGL((small_linear_rows_kernel<NC, TG, RQ, false>), grid, dim3(256), 0, st, a, g, eps);
+  return mm::check_launch("small_linear");
 }
 
 // Weight rows per workgroup: more of them read the token rows less often, fewer give more workgroups. us at 4 | 8 | 16
 // rows: N = 4096, 6 rows of 1024 6.4 | 5.3 | 4.6; 3072 5.2 | 4.8 | 4.2; 2048, 16 rows of 2048 6.8 | 5.4 | 6.2; 1152, 3
 // rows of 896 3.2 | 2.9 | 3.3; 1024, 6 rows of 1024 2.5 | 2.7 | 3.3, of 4096 4.6 | 5.4 | 7.1.
-template <int NC, int TG, bool GLU>
+template <int NC, int TG>
 int launch_rows_tg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  if constexpr (GLU) {
-    return launch_rows_rq<NC, TG, 2, true>(a, g, eps, st);
-  } else {
-    const int64_t cus = mm::cu_count();
-    if constexpr (NC <= 4) {
-      if (a.N >= 12 * cus) return launch_rows_rq<NC, TG, 4, false>(a, g, eps, st);
-    }
-    if (a.N > 4 * cus) return launch_rows_rq<NC, TG, 2, false>(a, g, eps, st);
-    return launch_rows_rq<NC, TG, 1, false>(a, g, eps, st);
+  const int64_t cus = mm::cu_count();
+  if constexpr (NC <= 4) {
+    if (a.N >= 12 * cus) return launch_rows_rq<NC, TG, 4>(a, g, eps, st);
   }
+  if (a.N > 4 * cus) return launch_rows_rq<NC, TG, 2>(a, g, eps, st);
+  return launch_rows_rq<NC, TG, 1>(a, g, eps, st);
 }
 
-template <int NC, bool GLU>
+template <int NC>
 int launch_rows_nc(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  if (a.M <= 4) return launch_rows_tg<NC, 1, GLU>(a, g, eps, st);
-  if (a.M <= 8) return launch_rows_tg<NC, 2, GLU>(a, g, eps, st);
-  if constexpr (NC <= 4) return launch_rows_tg<NC, 4, GLU>(a, g, eps, st);
+  if (a.M <= 4) return launch_rows_tg<NC, 1>(a, g, eps, st);
+  if (a.M <= 8) return launch_rows_tg<NC, 2>(a, g, eps, st);
+  if constexpr (NC <= 4) return launch_rows_tg<NC, 4>(a, g, eps, st);
   return MM_ERR_ARG;
 }
 
@@ -437,12 +427,11 @@ bool rows_form(const LinArgs& a) {
   return a.ws < (1LL << 27) && mm::rsrc_fits((static_cast<int64_t>(a.M) * a.xs + a.K) * 2);
 }
 
-template <bool GLU>
 int launch_rows(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  if (a.K <= 512) return launch_rows_nc<1, GLU>(a, g, eps, st);
-  if (a.K <= 1024) return launch_rows_nc<2, GLU>(a, g, eps, st);
-  if (a.K <= 2048) return launch_rows_nc<4, GLU>(a, g, eps, st);
-  return launch_rows_nc<8, GLU>(a, g, eps, st);
+  if (a.K <= 512) return launch_rows_nc<1>(a, g, eps, st);
+  if (a.K <= 1024) return launch_rows_nc<2>(a, g, eps, st);
+  if (a.K <= 2048) return launch_rows_nc<4>(a, g, eps, st);
+  return launch_rows_nc<8>(a, g, eps, st);
 }
 
 // Rows longer than one pass: each wave computes GPW = 64/LPR rows at a time, R times; LPR lanes share one
@@ -545,8 +534,8 @@ extern "C" int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_ro
   MM_REQUIRE(N <= 0x7fffffffLL * 8, "small_linear: N too large");
   MM_REQUIRE(x && w && y, "small_linear: null pointer");
   const bool once = (act & MM_NORM_ROUND_ONCE) != 0;
-  const bool invariant = (act & MM_ROW_INVARIANT) != 0;
-  act &= ~(MM_NORM_ROUND_ONCE | MM_ROW_INVARIANT);
+  const bool any_order = (act & MM_ANY_SUM_ORDER) != 0;
+  act &= ~(MM_NORM_ROUND_ONCE | MM_ANY_SUM_ORDER);
   MM_REQUIRE(act == MM_ACT_NONE || act == MM_ACT_GELU_TANH || act == MM_ACT_SILU, "small_linear: unknown act %d", act);
   MM_REQUIRE((x_row_stride >= K || x_row_stride == 0) && w_row_stride >= K && y_row_stride >= N,
              "small_linear: row stride too small (x rows may also repeat one row, stride 0)");
@@ -565,7 +554,7 @@ extern "C" int mm_small_linear(const void* x, int64_t M, int64_t K, int64_t x_ro
               static_cast<const uint16_t*>(b), act, once, static_cast<const uint16_t*>(residual), res_row_stride,
               static_cast<uint16_t*>(y), y_row_stride};
     auto g = static_cast<const uint16_t*>(norm_g);
-    if (!invariant && rows_form(a)) return launch_rows<false>(a, g, norm_eps, st);
+    if (any_order && rows_form(a)) return launch_rows(a, g, norm_eps, st);
     // chunks per lane NC = ceil(nch / 64), rounded up to an instantiated size; at most 16 loads per lane
     // (rows per wave measured on MI355X: 2 at K = 896; at K = 2048 1 up to N = 2048, 2 from N = 16 per CU on,
     // where each wave's activation row (and norm weights) from L2 then serves two weight rows: one token,
@@ -622,7 +611,6 @@ extern "C" int mm_small_linear_glu(const void* x, int64_t M, int64_t K, int64_t 
             inter, w_row_stride, nullptr, MM_ACT_NONE, false, nullptr, 0, static_cast<uint16_t*>(y), y_row_stride};
   auto g = static_cast<const uint16_t*>(norm_g);
   hipStream_t st = MM_STREAM(stream);
-  if (rows_form(a)) return launch_rows<true>(a, g, norm_eps, st);
   const int64_t nch = K / 8;
   if (nch <= 64) return launch_glu<1>(a, g, norm_eps, st);
   if (nch <= 128) return launch_glu<2>(a, g, norm_eps, st);

@@ -182,6 +182,12 @@ def _fuse(mods, attr="weight"):
     return fused
 
 
+def _rows_linear(*args, **kw):
+    """small_linear on the matrix units: the rows of a tail's sequence always come together, so none has to keep the
+    bits that it would get alone."""
+    return small_linear(*args, row_invariant=False, **kw)
+
+
 class _Block:
     """One DiT / aggregator transformer block on the fused kernels (fast_talker.py:82-102):
     h = h + to_out(rope_attn(q|k|v(RMSNorm1(h)))); h = h + W2(GELU_tanh(W1(RMSNorm2(h)))), every bias, norm,
@@ -204,10 +210,10 @@ class _Block:
         self.w2, self.b2 = ff[2].weight, ff[2].bias
 
     def __call__(self, h, cos, sin):
-        att = rope_attn(small_linear(h, self.wqkv, self.bqkv, norm=self.n1), cos, sin, self.heads)
-        h = small_linear(att, self.wo, self.bo, residual=h)
-        f = small_linear(h, self.w1, self.b1, act=1, norm=self.n2)
-        return small_linear(f, self.w2, self.b2, residual=h)
+        att = rope_attn(_rows_linear(h, self.wqkv, self.bqkv, norm=self.n1), cos, sin, self.heads)
+        h = _rows_linear(att, self.wo, self.bo, residual=h)
+        f = _rows_linear(h, self.w1, self.b1, act=1, norm=self.n2)
+        return _rows_linear(f, self.w2, self.b2, residual=h)
 
 
 def _rope_tables(rotary, n):
@@ -264,11 +270,11 @@ class FastTail:
         hs[:, :, 1] = small_linear(hist.reshape(1, -1), self.x_w, self.x_b)
         y = noise.reshape(1, -1)
         for i, dt in enumerate(self.dts):
-            small_linear(y.expand(2, -1), self.x_w, self.x_b, out=hs[i, :, 2])  # both rows at once
+            _rows_linear(y.expand(2, -1), self.x_w, self.x_b, out=hs[i, :, 2])  # both rows at once
             h = hs[i]
             for blk in self.blocks:
                 h = blk(h, self.cos3, self.sin3)
-            out = small_linear(h[:, -1], self.f_w, self.f_b, norm=self.f_norm)  # [2, latent]: pred, null
+            out = _rows_linear(h[:, -1], self.f_w, self.f_b, norm=self.f_norm)  # [2, latent]: pred, null
             y = cfg_update(y, out, self.cfg, dt)  # y + (pred + (pred - null) * cfg) * dt
         Da = self.a_x_w.shape[0]
         a = torch.stack([self.cls.reshape(1, Da), small_linear(y, self.a_x_w, self.a_x_b)], 1)  # [1, 2, Da]

@@ -70,11 +70,12 @@ def _launch(lib, x2, w, b, r2, act, norm, y, xn):
                                   _mm.ptr(xn), _mm.ptr(y), y.stride(0), _mm.stream_of(x2)), "small_linear")
 
 
-def small_linear(x, w, b=None, act=0, residual=None, out=None, norm=None, row_invariant=False):
+def small_linear(x, w, b=None, act=0, residual=None, out=None, norm=None, row_invariant=True):
     """x: [..., K] bf16; w: [N, K] contiguous; act: 0 none, 1 gelu-tanh, 2 silu;
     residual: tensor broadcastable as [..., N] added after the activation;
-    norm: (gamma, eps) applies RMSNorm to x first (fused); row_invariant: each row gets the bits that it gets alone
-    (several rows otherwise take the matrix units, whose fp32 sums run in another order)."""
+    norm: (gamma, eps) applies RMSNorm to x first (fused); row_invariant: each row gets the bits that it gets alone,
+    whatever rows come with it, up to the norm's rounding past MAX_M rows (False: several rows may take the matrix
+    units, whose fp32 sums run in another order)."""
     g = norm[0] if norm is not None else None
     _mm.require_gpu(x, w, b, residual, out, g)
     shape = x.shape
@@ -105,8 +106,8 @@ def small_linear(x, w, b=None, act=0, residual=None, out=None, norm=None, row_in
     xn = torch.empty(min(M, MAX_M), K, device=x.device, dtype=torch.bfloat16) if norm is not None and K > 8192 else None
     if M > MAX_M and norm is not None:
         act = int(act) | _mm.MM_NORM_ROUND_ONCE  # F.rms_norm's single rounding (fastlinear.py:151-153)
-    if row_invariant:
-        act = int(act) | _mm.MM_ROW_INVARIANT
+    if not row_invariant:
+        act = int(act) | _mm.MM_ANY_SUM_ORDER
     lib = _mm.load()
     with _mm.on_device(x):
         for m0 in range(0, M, MAX_M):

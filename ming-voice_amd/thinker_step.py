@@ -251,7 +251,7 @@ class FastThinkerStep:
         in_place: the residual is a buffer nobody reads afterwards, so the GEMM accumulates into it (beta = 1 on C = D,
         the same single rounding) instead of first copying it into a new output."""
         if x.shape[0] <= fastlinear.MAX_M:
-            return fastlinear.small_linear(x, w, b=b, residual=residual, norm=norm, row_invariant=True)
+            return fastlinear.small_linear(x, w, b=b, residual=residual, norm=norm)
         if norm is not None:
             x = fused_ops.rms_norm(x, norm[0], norm[1])
         if residual is not None and b is None:

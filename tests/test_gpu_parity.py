@@ -720,10 +720,10 @@ def test_small_linear(M, KN):
 @pytest.mark.parametrize("M,K,N", [(2, 8, 1), (3, 504, 5), (4, 512, 1023), (5, 520, 1029), (8, 1016, 3073), (9, 1024, 3075),
                                    (16, 2048, 2051), (8, 2056, 1026), (8, 4096, 1029), (9, 2056, 9), (8, 4104, 9)])
 def test_small_linear_rows_edges(M, K, N):
-    """Several rows on the matrix units: token groups of 4, weight rows 4, 8 and 16 to a workgroup with a remainder, k
-    chunks that end inside a wave's share, and the first shapes past it; bias, activation, residual, norm (both
-    roundings), rows with a stride or repeated, and the gated pair, which equals the two projections bit for bit. Sums of
-    K products in fp32: K 2^-24 of the sum of the magnitudes, and the bf16 rounding of the result."""
+    """Several rows, on the vector units and on the matrix units (row_invariant=False): token groups of 4, weight rows 4, 8
+    and 16 to a workgroup with a remainder, k chunks that end inside a wave's share, and the first shapes past it; bias,
+    activation, residual, norm, rows with a stride or repeated, and the gated pair, which equals the two projections bit
+    for bit. Sums of K products in fp32: K 2^-24 of the sum of the magnitudes, and the bf16 rounding of the result."""
     print(f"[small_linear rows] M={M} K={K} N={N}", flush=True)
     x = W.normal((M, K + 8), 1.0, 130 + M, DEV)[:, :K]  # strided rows
     w = W.normal((N, K), 0.05, 131, DEV)
@@ -735,11 +735,12 @@ def test_small_linear_rows_edges(M, K, N):
         mag = xin.double().abs() @ w.double().abs().t()
         bound = (K + 8) * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs() + 1e-30
         assert ((y.double() - want).abs() <= bound).all()
-    near(fastlinear.small_linear(x, w), x)
     one = x[:1].expand(M, -1)  # the same row M times: stride 0
-    near(fastlinear.small_linear(one, w), one)
-    y = fastlinear.small_linear(x, w, b, act=1, residual=r, norm=(g, 1e-6))
-    close(y, O.small_linear(x.cpu(), w.cpu(), b.cpu(), 1, r.cpu(), norm=(g.cpu(), 1e-6)))
+    want = O.small_linear(x.cpu(), w.cpu(), b.cpu(), 1, r.cpu(), norm=(g.cpu(), 1e-6))
+    for alone in (True, False):
+        near(fastlinear.small_linear(x, w, row_invariant=alone), x)
+        near(fastlinear.small_linear(one, w, row_invariant=alone), one)
+        close(fastlinear.small_linear(x, w, b, act=1, residual=r, norm=(g, 1e-6), row_invariant=alone), want)
     if N % 2 == 1:
         wgu = W.normal((2 * N, K), 0.05, 135, DEV)
         import fast_talker as FT
@@ -747,15 +748,22 @@ def test_small_linear_rows_edges(M, K, N):
                            FT.silu_mul(fastlinear.small_linear(x, wgu, norm=(g, 1e-6))))
 
 
-@pytest.mark.parametrize("M,K,N", [(2, 128, 2048), (7, 2048, 6416), (16, 2048, 2050), (5, 4096, 33)])
+@pytest.mark.parametrize("M,K,N", [(2, 128, 2048), (7, 2048, 6416), (16, 2048, 2050), (5, 4096, 33), (2, 512, 1152),
+                                   (3, 1024, 130), (16, 6144, 64), (4, 9216, 40)])
 def test_small_linear_row_invariant(M, K, N):
-    """row_invariant=True: each of M rows equals its own one-row call bit for bit (norm, bias and residual included)."""
+    """Each of M rows equals its own one-row call bit for bit (norm, bias and residual included), asked for or not, and so
+    does each row of the gated pair."""
+    import fast_talker as FT
     x, w = W.normal((M, K), 1.0, 150, DEV), W.normal((N, K), 0.05, 151, DEV)
     b, r, g = W.normal((N,), 1.0, 152, DEV), W.normal((M, N), 1.0, 153, DEV), W.normal((K,), 0.02, 154, DEV, mean=1.0)
     print(f"[small_linear row invariant] M={M} K={K} N={N}", flush=True)
-    y = fastlinear.small_linear(x, w, b, residual=r, norm=(g, 1e-6), row_invariant=True)
+    y = fastlinear.small_linear(x, w, b, residual=r, norm=(g, 1e-6))
+    assert torch.equal(y, fastlinear.small_linear(x, w, b, residual=r, norm=(g, 1e-6), row_invariant=True))
+    glu = FT.gate_up_silu(x, w[:N // 2 * 2], norm=(g, 1e-6)) if K <= 8192 else None
     for m in range(M):
         assert torch.equal(y[m:m + 1], fastlinear.small_linear(x[m:m + 1], w, b, residual=r[m:m + 1], norm=(g, 1e-6)))
+        if glu is not None:
+            assert torch.equal(glu[m:m + 1], FT.gate_up_silu(x[m:m + 1], w[:N // 2 * 2], norm=(g, 1e-6)))
 
 
 def test_small_linear_lm_head_shape():
