@@ -13,6 +13,8 @@
 // 64-wide slabs of the activation rows and of the weight rows straight into LDS (global_load_lds, several
 // slabs in flight) and feeds v_mfma_f32_16x16x32_bf16 from there. int8 weights stay int8 in LDS and are
 // widened to bf16 (exact for |q| <= 127) as fragments are read.
+#include <cmath>
+
 #include "mm_common.h"
 #include "mm_select.h"
 
@@ -210,7 +212,7 @@ struct LoadMap {
 // Issues the direct loads of slab kt into LDS stage `st` (arow/brow: this thread's source row starts,
 // null for masked rows; k counted in elements; slab kt of an activation row starts kt * aslab elements in, of a
 // weight row kt * bslab). ONCE && once: no other tile reads these weights, and keeping them in the caches would only push
-// out what others share (few_pairs).
+// out what others share (read_once).
 template <class G, bool ONCE>
 __device__ __forceinline__ void issue_slab(char* lds, int st, int kt, int64_t K, const LoadMap<G>& m,
                                            const uint16_t* const* arow, const char* const* brow, int64_t aslab,
@@ -644,28 +646,53 @@ int launch_down(const PrefillArgs& a, int64_t nb, hipStream_t st) {
   return mm::check_launch("moe_prefill down");
 }
 
-// Experts averaging few pairs mostly have one block, so that a tile's weight rows are no other's: the variants that load
-// those past the caches (ONCE). Above, most weights are shared, and the test alone costs the kernels 2 %. Block us with |
-// without: 64 experts, 4 / 16 / 28 pairs each 180 | 194, 215 | 229, 232 | 247, int8 110 | 114, 136 | 145; 38 / 43 / 48
-// 238 | 248, 240 | 246, 243 | 246; 55 247 | 246, int8 110 252 | 241; 128 experts, 21 / 35 / 49 152 | 162, 154 | 165,
-// 165 | 172. (For every tile's weights, shared or not, 512 tokens took 265 us instead of 248.)
-bool few_pairs(const PrefillArgs& a) { return a.P < static_cast<int64_t>(48) * a.E1; }
+// Whether a GEMM's weights are read past the caches (ONCE). Experts averaging few pairs mostly have one block, so that a
+// tile's weight rows are no other's: above, most weights are shared, and the test alone costs the kernels 2 %. A load has
+// to take whole lines of 128 bytes (the copies' pieces; bf16 rows at 128-byte strides): a line that the next slab reads
+// the rest of, as with int8 rows, would be fetched twice. And the stack has to be an eighth more than the 256 MB that the
+// last-level cache keeps from one pass to the next, and the part of it that P pairs reach, experts being alike, more than
+// these. Block us without | with, one layer in a loop, and layers in turn: 64 experts of 2048 x 1408 (1125 MB, int8 562), 9 /
+// 37 / 200 tokens 154 | 142, 213 | 198, 226 | 211 and 158 | 148, 214 | 199, 227 | 213; int8 copies 98 | 95, 132 | 121,
+// 144 | 134 and 99 | 96, 133 | 122, 145 | 136; int8 rows 99 | 120, 141 | 178, 158 | 203 and 106 | 127, 142 | 181, 159 | 203.
+// 128 experts of 1536 x 512 in int8 copies (304 MB, 142, 204, 281 and 304 of them reached), 9 / 16 / 37 / 100: 63 | 66, 70 | 72,
+// 81 | 80, 105 | 97 and 69 | 67, 75 | 73, 87 | 81, 107 | 98. 32 of 2048 x 704 (285 MB), 9 / 24 / 100: 63 | 74, 71 | 74, 77 | 78
+// and 70 | 67, 77 | 73, 81 | 79. Rows of 1000 elements, 37 tokens 132 | 133 and 126 | 130. int8 with fewer than two tiles a
+// CU gains nothing: 32 experts of 4096 x 1408 (363 gate/up tiles), 37 / 200 tokens 145 | 143, 158 | 163 and 146 | 147, 159 |
+// 165; 16 of 4096 x 2816 (374), 165 | 168, 172 | 184 and 167 | 169, 175 | 186; but 32 of 4096 x 2048 (528), 203 | 191, 206 | 200
+// and 205 | 192, 207 | 204. (Every tile's weights, shared or not: 512 tokens 248 -> 265 us.)
+bool read_once(const PrefillArgs& a, bool int8, const void* w, bool slabs, int64_t se, int64_t sn, int64_t nt) {
+  constexpr int64_t kLine = 128, kCache = 256 << 20;
+  if (a.P >= 48LL * a.E1 || reinterpret_cast<uintptr_t>(w) % kLine) return false;
+  const int64_t es = int8 ? 1 : 2;
+  if (!slabs && (int8 || se * es % kLine || sn * es % kLine)) return false;
+  if (int8 && a.E1 * nt < 2LL * mm::cu_count()) return false;
+  const int64_t stack = a.E1 * 3 * a.H * a.I * es;
+  const double reached = -std::expm1(-static_cast<double>(a.P) / a.E1) * static_cast<double>(stack);
+  return stack > kCache / 8 * 9 && reached > static_cast<double>(kCache);
+}
 
-template <bool Q, int BM, bool ONCE>
+template <bool Q, int BM>
 int launch_gemms(const PrefillArgs& a, int64_t nb, int phases, hipStream_t st) {
   constexpr int GU_BN = Q ? MM_PREFILL_GU_BN_INT8 : MM_PREFILL_GU_BN_BF16;
   constexpr int DOWN_BN = Q ? MM_PREFILL_DOWN_BN_INT8 : MM_PREFILL_DOWN_BN_BF16;
   constexpr int GU_NW = Q ? MM_PREFILL_GU_WAVES_INT8 : MM_PREFILL_GU_WAVES_BF16;
   constexpr int DOWN_NW = Q ? MM_PREFILL_DOWN_WAVES_INT8 : MM_PREFILL_DOWN_WAVES_BF16;
+  constexpr bool kOnce = BM == kBMSmall;  // blocks of kBM rows are for experts with many pairs
   int rc;
   if (phases & MM_PHASE_GATE_UP) {
-    rc = a.gu_slabs ? launch_gate_up<Q, GU_BN, GU_NW, BM, true, ONCE>(a, nb, st)
-                    : launch_gate_up<Q, GU_BN, GU_NW, BM, false, ONCE>(a, nb, st);
+    const bool once = kOnce && read_once(a, Q, a.w_gu, a.gu_slabs, a.gu_se, a.gu_sn, (2 * a.I + GU_BN - 1) / GU_BN);
+    if (a.gu_slabs) rc = once ? launch_gate_up<Q, GU_BN, GU_NW, BM, true, kOnce>(a, nb, st)
+                              : launch_gate_up<Q, GU_BN, GU_NW, BM, true, false>(a, nb, st);
+    else rc = once ? launch_gate_up<Q, GU_BN, GU_NW, BM, false, kOnce && !Q>(a, nb, st)
+                   : launch_gate_up<Q, GU_BN, GU_NW, BM, false, false>(a, nb, st);
     if (rc) return rc;
   }
   if (phases & MM_PHASE_DOWN) {
-    rc = a.d_slabs ? launch_down<Q, DOWN_BN, DOWN_NW, BM, true, ONCE>(a, nb, st)
-                   : launch_down<Q, DOWN_BN, DOWN_NW, BM, false, ONCE>(a, nb, st);
+    const bool once = kOnce && read_once(a, Q, a.w_d, a.d_slabs, a.d_se, a.d_sn, (a.H + DOWN_BN - 1) / DOWN_BN);
+    if (a.d_slabs) rc = once ? launch_down<Q, DOWN_BN, DOWN_NW, BM, true, kOnce>(a, nb, st)
+                             : launch_down<Q, DOWN_BN, DOWN_NW, BM, true, false>(a, nb, st);
+    else rc = once ? launch_down<Q, DOWN_BN, DOWN_NW, BM, false, kOnce && !Q>(a, nb, st)
+                   : launch_down<Q, DOWN_BN, DOWN_NW, BM, false, false>(a, nb, st);
     if (rc) return rc;
   }
   return MM_OK;
@@ -825,11 +852,9 @@ extern "C" int mm_moe_prefill(const void* x, int64_t n_tokens, int64_t x_row_str
   hipStream_t st = MM_STREAM(stream);
   if (phases == MM_PHASE_ALL) phases = MM_PHASE_GATE_UP | MM_PHASE_DOWN | MM_PHASE_COMBINE;
   if (nb > 0) {
-    const bool few = few_pairs(a);
-    if (ex->w_dtype == MM_INT8)
-      rc = few ? launch_gemms<true, kBMSmall, true>(a, nb, phases, st) : launch_gemms<true, kBMSmall, false>(a, nb, phases, st);
-    else if (block_m == kBM) rc = launch_gemms<false, kBM, false>(a, nb, phases, st);
-    else rc = few ? launch_gemms<false, kBMSmall, true>(a, nb, phases, st) : launch_gemms<false, kBMSmall, false>(a, nb, phases, st);
+    if (ex->w_dtype == MM_INT8) rc = launch_gemms<true, kBMSmall>(a, nb, phases, st);
+    else if (block_m == kBM) rc = launch_gemms<false, kBM>(a, nb, phases, st);
+    else rc = launch_gemms<false, kBMSmall>(a, nb, phases, st);
     if (rc) return rc;
   }
   if (!(phases & MM_PHASE_COMBINE)) return MM_OK;
