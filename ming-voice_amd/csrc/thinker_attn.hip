@@ -1524,6 +1524,37 @@ __global__ __launch_bounds__(256) void mla_split_kernel(MlaArgs a) {
 // the attention of 16 heads x (192, 128) took 15.1 us behind 2000 positions and 28.9 behind 4000; now 10.7 and 14.2.
 constexpr int kMergeBatch = 8;  // chunks per wave loaded ahead: 4 waves x 8 x 32 positions = 1024 positions
 constexpr int kMergeTail = 16;  // and per further batch: 2048 positions
+constexpr int kMergeFew = 4;    // where these are all: up to 1536 positions (16 loads for a chunk or two cost 0.2-0.4 us: the
+                                // attention of 16 heads x 64 at position 1100, 7.2 -> 6.7 us)
+
+// B chunks of the wave from c0 on (c0 + 4 b) into the running sums, every load in front of its first use.
+template <int NDV, int B>
+__device__ __forceinline__ void mla_merge_batch(const MlaArgs& a, const float* base, int64_t cs, int c0, int n, float m,
+                                                float (&acc)[NDV], float& l) {
+  const int lane = lane_id();
+  float tm[B], tl[B], tv[B][NDV];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const float* p = base + static_cast<int64_t>(min(c0 + 4 * b, n - 1)) * cs;
+    tm[b] = p[a.dv];
+    tl[b] = p[a.dv + 1];
+#pragma unroll
+    for (int j = 0; j < NDV; ++j) tv[b][j] = p[min(lane + kWave * j, a.dv - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    if (c0 + 4 * b < n) {  // uniform
+      const float wgt = __expf(tm[b] - m);
+      l = fmaf(tl[b], wgt, l);
+#pragma unroll
+      for (int j = 0; j < NDV; ++j) {
+        const int d = lane + kWave * j;
+        if (d < a.dv) acc[j] = fmaf(tv[b][j], wgt, acc[j]);
+      }
+    }
+  }
+}
 
 template <int NDV>
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaArgs a) {
@@ -1570,29 +1601,11 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaArgs a) {
       }
     }
   }
-  for (int c0 = wave + 4 * kMergeBatch; c0 < n; c0 += 4 * kMergeTail) {
-    float tm[kMergeTail], tl[kMergeTail], tv[kMergeTail][NDV];
-#pragma unroll
-    for (int b = 0; b < kMergeTail; ++b) {
-      const float* p = base + static_cast<int64_t>(min(c0 + 4 * b, n - 1)) * cs;
-      tm[b] = p[a.dv];
-      tl[b] = p[a.dv + 1];
-#pragma unroll
-      for (int j = 0; j < NDV; ++j) tv[b][j] = p[min(lane + kWave * j, a.dv - 1)];
-    }
-    __builtin_amdgcn_sched_barrier(0);  // every load of the batch in front of its first use
-#pragma unroll
-    for (int b = 0; b < kMergeTail; ++b) {
-      if (c0 + 4 * b < n) {  // uniform
-        const float wgt = __expf(tm[b] - m);
-        l = fmaf(tl[b], wgt, l);
-#pragma unroll
-        for (int j = 0; j < NDV; ++j) {
-          const int d = lane + kWave * j;
-          if (d < a.dv) acc[j] = fmaf(tv[b][j], wgt, acc[j]);
-        }
-      }
-    }
+  const int c1 = wave + 4 * kMergeBatch;
+  if (n <= 4 * (kMergeBatch + kMergeFew)) {
+    if (c1 < n) mla_merge_batch<NDV, kMergeFew>(a, base, cs, c1, n, m, acc, l);
+  } else {
+    for (int c0 = c1; c0 < n; c0 += 4 * kMergeTail) mla_merge_batch<NDV, kMergeTail>(a, base, cs, c0, n, m, acc, l);
   }
 #pragma unroll
   for (int j = 0; j < NDV; ++j) s_acc[wave][lane + kWave * j] = acc[j];

@@ -335,10 +335,10 @@ def test_mla_decode_attn_matches_oracle(nh, dq, dv, L):
 
 
 @pytest.mark.parametrize("nh,dq,dv", [(2, 192, 128), (1, 32, 40), (1, 64, 256)])
-@pytest.mark.parametrize("pos", [1023, 1024, 1151, 1152, 3071, 3072, 3199])
+@pytest.mark.parametrize("pos", [1023, 1024, 1151, 1152, 1535, 1536, 3071, 3072, 3199])
 def test_mla_decode_attn_at_the_edges_of_the_merge_batches(nh, dq, dv, pos):
-    """The merge takes 8 chunks of 32 positions per wave at first (up to 1023), then 16 per wave (up to 3071, ...);
-    a workspace of NaN shows that no chunk past the position enters."""
+    """The merge takes 8 chunks of 32 positions per wave at first (up to 1023), then 4 per wave where that is all (up to
+    1535), else 16 per wave (up to 3071, ...); a workspace of NaN shows that no chunk past the position enters."""
     kc = W.normal((1, nh, 3200, dq), 1.0, 422, DEV)
     vc = W.normal((1, nh, 3200, dv), 1.0, 423, DEV)
     q, kn, vn = W.normal((nh, dq), 1.0, 424, DEV), W.normal((nh, dq), 1.0, 425, DEV), W.normal((nh, dv), 1.0, 426, DEV)
