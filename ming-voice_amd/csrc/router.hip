@@ -121,29 +121,29 @@ __global__ __launch_bounds__(256) void router_gemv_kernel(const typename TX::T* 
 }
 
 // The same for bf16 rows of at most 2048 * J elements (H a multiple of 8, 16-byte aligned rows), in one
-// memory round trip, a workgroup per expert and token (grid (E, tokens)): thread i owns the 8-element chunks
+// memory round trip, a workgroup per expert and NT tokens (grid (E, tokens / NT)): thread i owns the 8-element chunks
 // i + 256 j, and every load of the workgroup (its router row, the RMSNorm weight, the token row) is issued at
 // kernel start through buffer resources. The sum of squares runs over the chunks exactly as row_rstd256 does, so
 // xn matches mm_rms_norm bit for bit; a chunk's logit terms are added in element order, chunks in j order, then
 // the waves in order. Bound by its chain (load, norm, dot), so every token takes its own workgroup, the router
 // rows coming from cache: a decode block of 5 / 7 tokens 22.0 / 25.2 us with 8 tokens to a workgroup, 20.5 / 22.9
-// with 2, 20.1 / 22.5 with one (64 experts of a tiny inner size, so that the front is what counts).
-template <int J>
+// with 2, 20.1 / 22.5 with one (64 experts of a tiny inner size, so that the front is what counts). Two tokens to a
+// workgroup from 12 workgroups a CU on, where the router rows read again count (launch_logits).
+template <int J, int NT>
 __global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* __restrict__ x, int64_t H, int64_t xs,
-                                                               const float* __restrict__ w32, int E,
+                                                               int n_tokens, const float* __restrict__ w32, int E,
                                                                float* __restrict__ logits,
                                                                const uint16_t* __restrict__ norm_w, float eps,
                                                                uint16_t* __restrict__ xn_out) {
-  __shared__ float red_ss[4];
-  __shared__ float red[4];
+  __shared__ float red_ss[NT][4];
+  __shared__ float red[NT][4];
   const int e = blockIdx.x;
-  const int64_t t = blockIdx.y;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * NT;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   const int nch = static_cast<int>(H / 8);
   const rsrc_t wr = make_rsrc(w32 + static_cast<int64_t>(e) * H, H * 4);
-  const rsrc_t xr = make_rsrc(x + t * xs, H * 2);
   const rsrc_t nr = make_rsrc(norm_w, norm_w ? H * 2 : 0);
-  uint4 wv[J][2], nv[J], xv[J];
+  uint4 wv[J][2], nv[J], xv[NT][J];
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int c = tid + 256 * j;
@@ -151,44 +151,65 @@ __global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* _
     wv[j][0] = buf16(wr, ok ? static_cast<uint32_t>(c) * 32u : kPast);
     wv[j][1] = buf16(wr, ok ? static_cast<uint32_t>(c) * 32u + 16u : kPast);
     nv[j] = buf16(nr, ok ? static_cast<uint32_t>(c) * 16u : kPast);
-    xv[j] = buf16(xr, ok ? static_cast<uint32_t>(c) * 16u : kPast);
-  }
-  float rstd = 1.f;
-  if (norm_w) {
-    float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < J; ++j) ss = chunk_ss_bf16x8(xv[j], ss);
-    ss = wave_sum(ss);
-    if (lane == 0) red_ss[wave] = ss;
+    for (int u = 0; u < NT; ++u) {  // a token past the last reads the last one's row and is not stored
+      const rsrc_t xr = make_rsrc(x + min(t0 + u, static_cast<int64_t>(n_tokens - 1)) * xs, H * 2);
+      xv[u][j] = buf16(xr, ok ? static_cast<uint32_t>(c) * 16u : kPast);
+    }
+  }
+  float rstd[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) rstd[u] = 1.f;
+  if (norm_w) {
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < J; ++j) ss = chunk_ss_bf16x8(xv[u][j], ss);
+      ss = wave_sum(ss);
+      if (lane == 0) red_ss[u][wave] = ss;
+    }
     __syncthreads();
-    rstd = rsqrtf((((red_ss[0] + red_ss[1]) + red_ss[2]) + red_ss[3]) / static_cast<float>(H) + eps);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      rstd[u] = rsqrtf((((red_ss[u][0] + red_ss[u][1]) + red_ss[u][2]) + red_ss[u][3]) / static_cast<float>(H) + eps);
   }
   const bool store_xn = xn_out && e == 0;
-  float acc = 0.f;
+  float acc[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) acc[u] = 0.f;
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int c = tid + 256 * j;
     const uint32_t wq[8] = {wv[j][0].x, wv[j][0].y, wv[j][0].z, wv[j][0].w, wv[j][1].x, wv[j][1].y, wv[j][1].z, wv[j][1].w};
     const uint32_t nq[4] = {nv[j].x, nv[j].y, nv[j].z, nv[j].w};
-    const uint32_t xq[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-    uint32_t o[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float lo = __uint_as_float(xq[i] << 16), hi = __uint_as_float(xq[i] & 0xffff0000u);
-      if (norm_w) {
-        lo = round_bf16(__uint_as_float(nq[i] << 16) * round_bf16(lo * rstd));
-        hi = round_bf16(__uint_as_float(nq[i] & 0xffff0000u) * round_bf16(hi * rstd));
+    for (int u = 0; u < NT; ++u) {
+      const uint32_t xq[4] = {xv[u][j].x, xv[u][j].y, xv[u][j].z, xv[u][j].w};
+      uint32_t o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float lo = __uint_as_float(xq[i] << 16), hi = __uint_as_float(xq[i] & 0xffff0000u);
+        if (norm_w) {
+          lo = round_bf16(__uint_as_float(nq[i] << 16) * round_bf16(lo * rstd[u]));
+          hi = round_bf16(__uint_as_float(nq[i] & 0xffff0000u) * round_bf16(hi * rstd[u]));
+        }
+        o[i] = static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
+        acc[u] = fmaf(lo, __uint_as_float(wq[2 * i]), acc[u]);
+        acc[u] = fmaf(hi, __uint_as_float(wq[2 * i + 1]), acc[u]);
       }
-      o[i] = static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
-      acc = fmaf(lo, __uint_as_float(wq[2 * i]), acc);
-      acc = fmaf(hi, __uint_as_float(wq[2 * i + 1]), acc);
+      if (store_xn && c < nch && t0 + u < n_tokens)
+        reinterpret_cast<uint4*>(xn_out + (t0 + u) * H)[c] = make_uint4(o[0], o[1], o[2], o[3]);
     }
-    if (store_xn && c < nch) reinterpret_cast<uint4*>(xn_out + t * H)[c] = make_uint4(o[0], o[1], o[2], o[3]);
   }
-  acc = wave_sum(acc);
-  if (lane == 0) red[wave] = acc;
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    acc[u] = wave_sum(acc[u]);
+    if (lane == 0) red[u][wave] = acc[u];
+  }
   __syncthreads();
-  if (tid == 0) logits[t * E + e] = ((red[0] + red[1]) + red[2]) + red[3];
+  if (tid < NT && t0 + tid < n_tokens)
+    logits[(t0 + tid) * E + e] = ((red[tid][0] + red[tid][1]) + red[tid][2]) + red[tid][3];
 }
 
 // logits for many tokens on fp32 MFMA (v_mfma_f32_16x16x4_f32): a workgroup of 16 waves computes 16
@@ -430,10 +451,14 @@ int launch_logits(const void* x, int64_t n_tokens, int64_t H, int64_t xs, const 
                     n_tokens * xs * 2 < (1LL << 31);
   if (fast && n_tokens <= 8) {  // larger batches take the MFMA tiles, on normalised rows
     const auto* xb = static_cast<const uint16_t*>(x);
-    const dim3 grid(static_cast<unsigned>(E), static_cast<unsigned>(n_tokens));
-    const int e = static_cast<int>(E);
-    if (H <= 2048) hipLaunchKernelGGL(router_gemv_bf16_kernel<1>, grid, dim3(256), 0, s, xb, H, xs, w32, e, logits, nw, eps, xo);
-    else hipLaunchKernelGGL(router_gemv_bf16_kernel<2>, grid, dim3(256), 0, s, xb, H, xs, w32, e, logits, nw, eps, xo);
+    const int e = static_cast<int>(E), nt = static_cast<int>(n_tokens);
+    // logits and selection of 8 tokens, us with 1 | 2 | 8 tokens to a workgroup: 512 experts of 4096 12.7 | 11.8 | 12.0, of 2048
+    // 11.1 | 10.7 | 10.8; 256 of 4096 7.5 | - | 7.9; a single token 8.5 with any
+    const bool pairs = E * n_tokens >= 12LL * mm::cu_count();
+    const dim3 grid(static_cast<unsigned>(E), static_cast<unsigned>(pairs ? (n_tokens + 1) / 2 : n_tokens));
+    auto kern = H <= 2048 ? (pairs ? router_gemv_bf16_kernel<1, 2> : router_gemv_bf16_kernel<1, 1>)
+                          : (pairs ? router_gemv_bf16_kernel<2, 2> : router_gemv_bf16_kernel<2, 1>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, xb, H, xs, nt, w32, e, logits, nw, eps, xo);
   } else if (n_tokens <= 8) {
     hipLaunchKernelGGL(router_gemv_kernel<TX>, dim3(static_cast<unsigned>(E)), dim3(256), 0, s, xp,
                        static_cast<int>(n_tokens), H, xs, w32, static_cast<int>(E), logits, nw, eps, xo);

@@ -248,6 +248,25 @@ def test_moe_block_decode_matches_unfused_and_oracle(blk, n, int8):
     close(y, _oracle_moe(cpu, xn, ids, wts, int8=int8, residual=x.cpu()))
 
 
+@pytest.mark.parametrize("E,H,n", [(512, 2048, 5), (512, 2048, 6), (512, 2048, 7), (440, 4096, 7), (512, 4096, 8),
+                                   (384, 2056, 8), (511, 1000, 7)])
+def test_router_tokens_in_pairs(E, H, n):
+    """Batches of many experts put two tokens in a workgroup (from 12 workgroups a CU on; an odd last token by itself): the
+    logits equal each token's own call bit for bit, with and without the norm, and those of the normalised rows."""
+    print(f"[router pairs] E={E} H={H} n={n}", flush=True)
+    x, w32 = W.tokens(n, seed=160, device=DEV, hidden=H), W.normal((E, H), 0.02, 161, DEV, dtype=torch.float32)
+    nw = W.normal((H,), 0.02, 162, DEV, mean=1.0)
+    logits = fused_ops.route(x, w32, top_k=2)[2]
+    assert torch.equal(logits, torch.cat([fused_ops.route(x[i:i + 1], w32, top_k=2)[2] for i in range(n)]))
+    err, mag = (logits.double() - x.double() @ w32.double().t()).abs(), x.double().abs() @ w32.double().abs().t()
+    assert (err <= (H + 8) * 2.0 ** -24 * mag).all()
+    if H % 16 == 0:  # the block takes rows of whole 16-element pieces
+        w_gu, w_d = W.normal((E + 1, 32, H), 0.02, 163, DEV), W.normal((E + 1, H, 16), 0.02, 164, DEV)
+        _, ids, wts, got = fused_moe.moe_block_decode(x, nw, W.EPS, w32, w_gu, w_d, top_k=2)
+        want = fused_ops.route(fused_ops.rms_norm(x, nw, W.EPS), w32, top_k=2)
+        assert torch.equal(got, want[2]) and torch.equal(ids, want[0]) and torch.equal(wts, want[1])
+
+
 def test_moe_block_decode_sigmoid_group_thinker_router():
     """The Ming thinker's router (128 experts, 8 groups, top 4 groups, top 8, scale 2.5) on the fused path."""
     H, I, E = 1536, 512, 128
