@@ -92,7 +92,8 @@ def test_decode_attn_talker_shape(pos):
                                                    (12, 2, 128, 4096, 4000), (8, 4, 256, 300, 257),
                                                    (6, 2, 96, 129, 128), (7, 7, 64, 1, 0),
                                                    (14, 2, 64, 2048, 1500), (14, 2, 64, 1025, 1024),
-                                                   (4, 2, 32, 1024, 1023)])
+                                                   (4, 2, 32, 1024, 1023), (16, 1, 256, 200, 170),
+                                                   (26, 2, 224, 130, 129)])
 def test_decode_attn_shapes(nh, nkv, hd, max_len, pos):
     """Head dims 32-256, GQA groups 1-16, caches of 1 to 4096 positions (a partial last chunk, pos at a chunk
     edge and at the cache end)."""
