@@ -294,7 +294,8 @@ __global__ __launch_bounds__(256) void small_linear_rows_kernel(LinArgs a, const
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
     const int64_t row = n0 + 4 * q, left = a.N - row;  // its rows: 4 at most
-    const rsrc_t wr = make_rsrc(a.w + (left > 0 ? row : 0) * a.ws, left > 0 ? ((min(left, static_cast<int64_t>(4)) - 1) * a.ws + a.K) * 2 : 0);
+    const rsrc_t wr =
+        make_rsrc(a.w + (left > 0 ? row : 0) * a.ws, left > 0 ? ((min(left, static_cast<int64_t>(4)) - 1) * a.ws + a.K) * 2 : 0);
 #pragma unroll
     for (int j = 0; j < NC; ++j) wv[q][j] = buf16(wr, c16[j] == kPast ? kPast : static_cast<uint32_t>(r * a.ws) * 2u + c16[j]);
   }
@@ -400,10 +401,9 @@ int launch_rows_rq(const LinArgs& a, const uint16_t* g, float eps, hipStream_t s
 }
 
 // Weight rows per workgroup: more of them read the token rows less often, fewer give more workgroups (16 where these make
-// about one workgroup a CU, or many; in between a second round of them is nearly empty: 6 rows of 2048 -> 5120 with 8 | 16
-// 6.8 | 7.4). us at 4 | 8 | 16
-// rows: N = 4096, 6 rows of 1024 6.4 | 5.3 | 4.6; 3072 5.2 | 4.8 | 4.2; 2048, 16 rows of 2048 6.8 | 5.4 | 6.2; 1152, 3
-// rows of 896 3.2 | 2.9 | 3.3; 1024, 6 rows of 1024 2.5 | 2.7 | 3.3, of 4096 4.6 | 5.4 | 7.1.
+// about one workgroup a CU, or many; in between a second round of them is nearly empty). us at 4 | 8 | 16 rows: N = 5120, 6
+// rows of 2048 7.8 | 6.9 | 7.6; 4096, 6 rows of 1024 6.4 | 5.3 | 4.6; 3072 5.2 | 4.8 | 4.2; 2048, 16 rows of 2048 6.8 | 5.4 |
+// 6.2; 1152, 3 rows of 896 3.2 | 2.9 | 3.3; 1024, 6 rows of 1024 2.5 | 2.7 | 3.3, of 4096 4.6 | 5.4 | 7.1.
 template <int NC, int TG>
 int launch_rows_tg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
   const int64_t cus = mm::cu_count();
@@ -416,18 +416,20 @@ int launch_rows_tg(const LinArgs& a, const uint16_t* g, float eps, hipStream_t s
 
 template <int NC>
 int launch_rows_nc(const LinArgs& a, const uint16_t* g, float eps, hipStream_t st) {
-  if (a.M <= 4) return launch_rows_tg<NC, 1>(a, g, eps, st);
-  if (a.M <= 8) return launch_rows_tg<NC, 2>(a, g, eps, st);
-  if constexpr (NC <= 4) return launch_rows_tg<NC, 4>(a, g, eps, st);
-  return MM_ERR_ARG;
+  if constexpr (NC <= 4) {  // rows past 2048 elements: 6 to 8 of them (rows_form)
+    if (a.M <= 4) return launch_rows_tg<NC, 1>(a, g, eps, st);
+    if (a.M > 8) return launch_rows_tg<NC, 4>(a, g, eps, st);
+  }
+  return launch_rows_tg<NC, 2>(a, g, eps, st);
 }
 
 // Whether the matrix-unit form takes (M, K, N): its lanes hold all their chunks of the token rows at once, a row group
 // and the tokens are addressed by 32-bit offsets, and it is no slower than the vector form where the weights are in the
 // caches (from memory it is 5 to 35 % faster almost everywhere). us of the vector form | this one, weights in the caches:
-// 2 / 5 / 8 rows of 1024 -> 4096 3.5 | 3.2, 4.1 | 3.6, 4.7 | 3.7; 2048 -> 2048 3.4 | 3.2, 4.1 | 3.7, 4.7 | 4.0, -> 6416 4.9 | 6.4,
-// 6.9 | 7.4, 8.8 | 8.0; 4096 -> 1024 3.3 | 3.5, 4.1 | 4.2, 5.2 | 4.8 (6 rows 4.5 | 4.4), -> 4096 4.8 | 6.8, 7.3 | 8.2, 9.5 | 9.5; with the
-// norm, 5 / 8 / 16 rows of 2048 -> 64 4.0 | 4.5, 4.0 | 4.8, 4.0 | 6.7, 12 rows of 2048 -> 1024 5.9 | 6.6, of 1024 -> 64 4.4 | 4.7.
+// 2 / 5 / 8 rows of 1024 -> 4096 3.5 | 3.2, 4.1 | 3.6, 4.7 | 3.7; 2048 -> 2048 3.4 | 3.2, 4.1 | 3.7, 4.7 | 4.0, -> 6416
+// 4.9 | 6.4, 6.9 | 7.4, 8.8 | 8.0; 4096 -> 1024 3.3 | 3.5, 4.1 | 4.2, 5.2 | 4.8 (6 rows 4.5 | 4.4), -> 4096 4.8 | 6.8,
+// 7.3 | 8.2, 9.5 | 9.5; with the norm, 5 / 8 / 16 rows of 2048 -> 64 4.0 | 4.5, 4.0 | 4.8, 4.0 | 6.7, 12 rows of 2048 -> 1024
+// 5.9 | 6.6, of 1024 -> 64 4.4 | 4.7.
 bool rows_form(const LinArgs& a) {
   if (a.M < 2 || a.K > 4096 || (a.M > 8 && a.K > 2048)) return false;
   const int64_t cus = mm::cu_count();

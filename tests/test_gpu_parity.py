@@ -737,7 +737,8 @@ def test_small_linear(M, KN):
 
 
 @pytest.mark.parametrize("M,K,N", [(2, 8, 1), (3, 504, 5), (4, 512, 1023), (5, 520, 1029), (8, 1016, 3073), (9, 1024, 3075),
-                                   (16, 2048, 2051), (8, 2056, 1026), (8, 4096, 1029), (9, 2056, 9), (8, 4104, 9)])
+                                   (16, 2048, 2051), (8, 2056, 1026), (8, 4096, 1029), (9, 2056, 9), (8, 4104, 9),
+                                   (6, 4096, 1024), (3, 1032, 2045), (6, 2048, 5121), (7, 2048, 6147)])
 def test_small_linear_rows_edges(M, K, N):
     """Several rows, on the vector units and on the matrix units (row_invariant=False): token groups of 4, weight rows 4, 8
     and 16 to a workgroup with a remainder, k chunks that end inside a wave's share, and the first shapes past it; bias,
