@@ -302,18 +302,14 @@ __device__ __forceinline__ uint4 buf16(rsrc_t r, uint32_t off) {
 // For memory that a launch reads once, the weights of a decode step above all: the nt bit, with which the lines are not
 // kept in the caches (a step streams more weights than these hold, so that keeping them only pushes out what is read
 // again). Cold decode blocks, us per layer with | without: bf16 one token 28.2 | 29.7, int8 21.2 | 23.4, bf16 8 tokens
-// 96.9 | 104.4; a Talker token 545 | 601, a 4-layer int8 thinker token 265 | 287.
+// 96.9 | 104.4; a Talker token 574 | 601, a 4-layer int8 thinker token 265 | 287. Weights that the caches hold from one
+// launch to the next: one-row linears within 3 % either way, decode blocks 0.89 to 1.08 of the time without.
 __device__ __forceinline__ uint4 buf16_once(rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 2));
 }
 __device__ __forceinline__ uint4 ld16_once(const uint16_t* p) {
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
-}
-
-// With a wave-uniform part of the offset, which costs no vector instruction.
-__device__ __forceinline__ float4 buf16f(rsrc_t r, uint32_t off, uint32_t uniform) {
-  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), static_cast<int>(uniform), 0));
 }
 
 __device__ __forceinline__ uint32_t buf4(rsrc_t r, uint32_t off) {
