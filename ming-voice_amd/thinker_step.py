@@ -52,9 +52,9 @@ import thinker_attn as TA
 __all__ = ["FastThinkerStep"]
 
 _SCORING = ("sigmoid", "softmax")
-# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda), as the engine switches its KDA layers'
+# Prompts longer than this take the KDA recurrence in chunked form (chunk_kda), where the engine switches its KDA layers'
 # mode (engine.py:946-949, 964-967). us per layer's core at 32 / 64 / 150 / 192 / 512 rows: 12.2 / 14.3 / 20.1 / 21.9 /
-# 43.7 chunked, 13.9 / 19.7 / 35.4 / 40.9 / 92.4 recurrent; shorter prompts keep the recurrent form's bits.
+# 43.7 chunked, 13.9 / 19.7 / 35.4 / 40.9 / 92.4 recurrent: the chunked form is faster before, but sums in another order.
 KDA_CHUNK_ABOVE = 192
 
 
