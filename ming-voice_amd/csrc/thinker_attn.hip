@@ -2386,6 +2386,9 @@ extern "C" int mm_mla_prefill_attn(const void* q, int64_t q_ts, const void* k_ne
     int rc = mm::check_launch("mla_prefill_attn store");
     if (rc) return rc;
   }
+  // 192 in its 6 steps of 32; any other dqk in 8, the ones past it masked. us against a loop of dqk / 32 steps over tiles by
+  // register loads, 16 heads at 500@611 and 2000@2000: 64 / 64 19.6 | 48.7 and 125 | 476, 96 / 64 19.6 | 36.9 and 124 | 307,
+  // 128 / 128 23.3 | 59.8 and 147 | 579, 256 / 128 24.2 | 62.4 and 152 | 592
   if (dv <= 64)
     return dqk == 192 ? launch_mla_prefill_shape<6, true, 4>(a, st) : launch_mla_prefill_shape<8, false, 4>(a, st);
   return dqk == 192 ? launch_mla_prefill_shape<6, true, 8>(a, st) : launch_mla_prefill_shape<8, false, 8>(a, st);
