@@ -401,8 +401,9 @@ int mm_mla_decode_attn(const void* q, const void* k_new, const void* v_new, int 
  * scalar (MM_INT64 / MM_INT32), the first token's position. A prompt outside [0, max_len) (pos < 0 or
  * pos + T > max_len) writes nothing to the caches and sets out to NaN. dqk a multiple of 8 up to 256, dv a multiple of
  * 8 up to 128; q, k_new, v_new and the caches 16-byte aligned with rows at 16-byte strides, out 8-byte aligned. out
- * may lie over v_new or k_new (both are in the caches by then: one more launch), not over q or the caches. With
- * T = 1 it computes what mm_mla_decode_attn does. */
+ * may lie over v_new or k_new (both are in the caches by then: one more launch) and, with dqk = dv and q's own stride,
+ * over q (a workgroup reads its queries before it stores), not over the caches. With T = 1 it computes what
+ * mm_mla_decode_attn does. */
 int mm_mla_prefill_attn(const void* q, int64_t q_ts, const void* k_new, int64_t k_ts, const void* v_new, int64_t v_ts,
                         int64_t T, int nh, int dqk, int dv, void* k_cache, void* v_cache, int64_t max_len,
                         const void* pos, int pos_dtype, float scale, void* out, int64_t out_ts, void* stream);

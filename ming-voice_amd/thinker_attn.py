@@ -373,7 +373,7 @@ def mla_prefill_attn(q, k_new, v_new, k_cache, v_cache, pos, scale=None, out=Non
     pos: a one-element int64 / int32 device tensor, the first token's position. Writes the new rows at
     pos .. pos + T - 1 and returns out [T, nh * dv]: token t attends to positions 0 .. pos + t (scale defaults to
     dqk ** -0.5). A prompt that does not fit in the cache leaves it unchanged and returns NaN. out may lie over v_new
-    or k_new (the rows are then stored by a launch of their own), not over q or the caches."""
+    or k_new (the rows are then stored by a launch of their own) and, with dqk = dv, over q; not over the caches."""
     _mm.require_gpu(q, k_new, v_new, k_cache, v_cache, pos, out)
     nh, max_len, dqk = k_cache.shape[-3:]
     dv = v_cache.shape[-1]

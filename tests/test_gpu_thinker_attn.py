@@ -525,6 +525,19 @@ def test_mla_prefill_out_over_the_new_rows(T, pos, over):
     assert torch.equal(kc, k2) and torch.equal(vc, v2)
 
 
+@pytest.mark.parametrize("T,pos", [(33, 31), (300, 40), (544, 10)])
+def test_mla_prefill_out_over_the_queries(T, pos):
+    """out in the buffer of q (dqk = dv), for every shape of the workgroups: the result of a separate out, bit for bit."""
+    nh, d = 16, 128
+    print(f"[mla prefill out over q] T={T} pos={pos}", flush=True)
+    kc, vc = W.normal((1, nh, T + pos, d), 1.0, 560, DEV), W.normal((1, nh, T + pos, d), 1.0, 561, DEV)
+    q, kn, vn = (x.reshape(T, -1) for x in _prompt(nh, d, d, T, 562))
+    k2, v2, p = kc.clone(), vc.clone(), torch.tensor([pos], device=DEV)
+    want = TA.mla_prefill_attn(q, kn, vn, k2, v2, p)
+    assert torch.equal(TA.mla_prefill_attn(q, kn, vn, kc, vc, p, out=q), want)
+    assert torch.equal(kc, k2) and torch.equal(vc, v2)
+
+
 def test_mla_prefill_one_token_equals_decode_and_graph_replays_follow_the_position():
     nh, dq, dv, L = 16, 192, 128, 512
     kc = W.normal((1, nh, L, dq), 1.0, 520, DEV)
